@@ -295,7 +295,7 @@ def write_if_changed(path: Path, text: str):
 
 def sources():
     GEN.mkdir(parents=True, exist_ok=True)
-    srcs = [CSRC / "api.hip"]
+    srcs = [CSRC / "api.hip", CSRC / "life_packed.hip"]
     for st, ops in CATALOG:
         for ctype, code in FLOAT_TYPES:
             p = GEN / f"static_{shape_name(st)}_{ctype}.hip"

@@ -24,6 +24,7 @@
 #include "life2_kernel.hpp"
 #include "lifeb_kernel.hpp"
 #include "life_kernel.hpp"
+#include "lifep_kernel.hpp"
 #include "multi_kernel.hpp"
 #include "registry.hpp"
 #include "scatter_kernel.hpp"
@@ -150,6 +151,7 @@ struct Plan {
   int32_t jit_fused_3d;    // its grid: tiles_x * tiles_y (2-D) or * tiles_z (3-D)
   int32_t fused_gens;      // steps fn_fused advances per launch
   int32_t fused_tiles_x, fused_tiles_y, fused_tiles_z;  // its grid
+  int32_t life_packed;      // iterations may run on packed bits (lifep_kernel.hpp)
   HaloParams hp;
   void (*halo_fn)(const HaloParams&, hipStream_t);
 };
@@ -383,6 +385,12 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
   std::string group;
   const int64_t cells = n[0] * n[1] * n[2];
   auto ilog2 = [](int64_t v) { int r = 0; while (v > 1) { v >>= 1; ++r; } return r; };
+  // Life iterations on packed bits: any grid whose rows hold their own packed
+  // form (both buffers' rows are the iteration's to overwrite)
+  if (!(flags & (STH_GENERIC | STH_NO_FUSE)) && op->kind == STH_OP_LIFE && (sdt == STH_U8 || sdt == STH_BOOL) &&
+      moore1 && src->ndim == 2 && bc != STH_USE && n[0] >= kLifepMinN0 && n[1] >= 3 && n[0] < (int64_t(1) << 30) &&
+      n[1] < (int64_t(1) << 30) && p.src.s1 >= n[0] && p.dst.s1 >= n[0])
+    pl.life_packed = 1;
   const std::string bucket = "|c" + std::to_string(ilog2(cells)) + "|x" + std::to_string(ilog2(n[0]));
   if (!(flags & STH_GENERIC) && op->kind == STH_OP_LIFE && (sdt == STH_U8 || sdt == STH_BOOL) &&
       moore1 && src->ndim == 2 && n[0] % 16 == 0 && aligned16(p.src) && aligned16(p.dst)) {
@@ -1224,6 +1232,151 @@ static int clear_graphs(sth_ctx* ctx) {
   return STH_OK;
 }
 
+namespace {
+// Calls of a few launches go straight to the stream even with STH_GRAPH: a
+// graph launch costs the host about 27 us against about 16 us for six direct
+// launches, and the device is the bound either way (Life 8192^2, 20 steps:
+// 152 us direct, 159 us replayed).
+constexpr int64_t kGraphMinLaunches = 17;
+
+// Launches the graph that `enqueue(stream)` records, `times` times on `s`.
+// Graphs of an iteration's steps are captured once per parameter set (the
+// bytes of its two step plans, and `tag`: the step layout) and replayed.  The
+// lookup and the launches happen under ctx->mu, so a cache eviction on
+// another thread cannot destroy an executable between the two.
+template <class F>
+int replay_graph(sth_ctx* ctx, const Plan& ab, const Plan& ba, const std::string& tag, int64_t times, hipStream_t s,
+                 F&& enqueue) {
+  std::string key(reinterpret_cast<const char*>(&ab), sizeof(Plan));
+  key.append(reinterpret_cast<const char*>(&ba), sizeof(Plan));
+  key.append(tag);
+  std::lock_guard<std::mutex> lk(ctx->mu);
+  auto it = ctx->graphs.find(key);
+  if (it != ctx->graphs.end()) {
+    for (int64_t i = 0; i < times; ++i) STH_HIP(hipGraphLaunch(it->second, s));
+    return STH_OK;
+  }
+  STH_HIP(hipStreamBeginCapture(ctx->capture, hipStreamCaptureModeThreadLocal));
+  const int r2 = enqueue(ctx->capture);
+  hipGraph_t g = nullptr;
+  hipError_t e = hipStreamEndCapture(ctx->capture, &g);
+  if (r2) {
+    if (g) (void)hipGraphDestroy(g);
+    return r2;
+  }
+  if (e != hipSuccess) return fail(STH_EDEVICE, "hipStreamEndCapture: %s", hipGetErrorString(e));
+  hipGraphExec_t x = nullptr;
+  e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(g);
+  if (e != hipSuccess) return fail(STH_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e));
+  if (ctx->graphs.size() >= kMaxGraphs) {
+    // bound the cache (a long-running caller iterating ever new buffers
+    // would grow it without end): wait for the device, then drop it all
+    if (int r3 = clear_graphs(ctx)) {
+      (void)hipGraphExecDestroy(x);
+      return r3;
+    }
+  }
+  ctx->graphs.emplace(key, x);
+  for (int64_t i = 0; i < times; ++i) STH_HIP(hipGraphLaunch(x, s));
+  return STH_OK;
+}
+
+// Fewest steps of a Life iteration that run packed: pack, launches in pairs,
+// unpack and two single steps are then no more launches than the steps.
+constexpr int64_t kLifepMinSteps = 8;
+
+// A Life iteration of `steps` generations from the a -> b plan `ab` and the
+// b -> a plan `ba`, on packed bits (lifep_kernel.hpp): a's cells are packed
+// into b, F launches advance steps - 2 generations between the buffers, the
+// result is unpacked into the other buffer, and two single steps leave both
+// buffers and their halos as the step-by-step reference does.  F has the
+// parity of steps - 2, so those steps write the buffers they would write
+// step by step.  Every cell is 0 or 1 after the unpacking, as after a step.
+int iterate_life_packed(sth_ctx* ctx, const Plan& ab, const Plan& ba, int64_t steps, uint32_t flags, hipStream_t s) {
+  const MapParams& m = ab.p;
+  const bool conway = m.op.birth == (1ull << 3) && m.op.survive == ((1ull << 2) | (1ull << 3));
+  const LifepShape shape = lifep_shape(m.src.n0, m.src.n1, conway, ctx->cus);
+  const LifepFn launch = lifep_launcher(shape.k, conway, m.bc);
+  LifepParams q{};
+  q.n0 = static_cast<int32_t>(m.src.n0);
+  q.n1 = static_cast<int32_t>(m.src.n1);
+  q.words = lifep_words(m.src.n0);
+  q.pad = (m.padval & 0xffu) ? 0xffffffffu : 0u;
+  q.birth = static_cast<uint32_t>(m.op.birth & 0x1ffu);
+  q.survive = static_cast<uint32_t>(m.op.survive & 0x1ffu);
+  auto between = [&](bool a_to_b) {
+    const DevArr &x = a_to_b ? m.src : m.dst, &y = a_to_b ? m.dst : m.src;
+    q.src = x.base;
+    q.s1 = x.s1;
+    q.dst = y.base;
+    q.d1 = y.s1;
+    return q;
+  };
+  const int64_t gens = steps - 2, G = shape.gens;
+  int64_t F = (gens + G - 1) / G;
+  if ((F ^ gens) & 1) ++F;
+  // all launches but the last four take G generations, those four share the rest
+  const int64_t full = std::max<int64_t>(0, F - 4);
+  // launch i runs from b when i is even
+  auto advance = [&](hipStream_t st, int64_t i, int64_t g) -> int {
+    LifepParams l = between(i % 2 != 0);
+    l.gens = static_cast<int32_t>(g);
+    lifep_grid(l.n0, l.n1, shape.k, l.gens, &l.tiles_x, &l.tiles_y);
+    launch(l, st);
+    STH_HIP(hipGetLastError());
+    return STH_OK;
+  };
+  auto head = [&](hipStream_t st) -> int {
+    launch_life_pack(between(true), st);
+    STH_HIP(hipGetLastError());
+    return STH_OK;
+  };
+  auto tail = [&](hipStream_t st, int64_t from) -> int {
+    int r2 = STH_OK;
+    int64_t left = gens - from * G;
+    for (int64_t i = from; i < F && r2 == STH_OK; ++i) {
+      const int64_t g = i < full ? G : (left + (F - i) - 1) / (F - i);
+      left -= g;
+      r2 = advance(st, i, g);
+    }
+    if (r2) return r2;
+    launch_life_unpack(between(F % 2 != 0), st);
+    STH_HIP(hipGetLastError());
+    const Plan &p0 = F % 2 ? ba : ab, &p1 = F % 2 ? ab : ba;
+    if ((r2 = run_plan(p0, st, true))) return r2;
+    return run_plan(p1, st, true);
+  };
+  int rc;
+  const int64_t launches = F + 4;
+  if (!(flags & STH_GRAPH) || launches < kGraphMinLaunches) {
+    if ((rc = head(s))) return rc;
+    return tail(s, 0);
+  }
+  // graphs: 32 full launches (replayed), then the rest of the call
+  constexpr int64_t FU = 32;
+  const int64_t reps = full / FU;
+  auto tag = [](const char* t, int64_t x, int64_t y) {
+    return std::string(t) + std::to_string(x) + "," + std::to_string(y);
+  };
+  if (reps == 0)
+    return replay_graph(ctx, ab, ba, tag("lh", gens, 0), 1, s, [&](hipStream_t st) -> int {
+      const int r2 = head(st);
+      return r2 ? r2 : tail(st, 0);
+    });
+  if ((rc = head(s))) return rc;
+  if ((rc = replay_graph(ctx, ab, ba, tag("lb", G, FU), reps, s, [&](hipStream_t st) -> int {
+         int r2 = STH_OK;
+         for (int64_t i = 0; i < FU && r2 == STH_OK; ++i) r2 = advance(st, i, G);
+         return r2;
+       })))
+    return rc;
+  return replay_graph(ctx, ab, ba, tag("lt", gens - reps * FU * G, F - reps * FU), 1, s,
+                      [&](hipStream_t st) { return tail(st, reps * FU); });
+}
+
+}  // namespace
+
 extern "C" {
 
 int sth_version(void) { return STH_ABI_VERSION * 10000 + 0; }
@@ -1891,6 +2044,11 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
   }
   *current = static_cast<int32_t>(steps % 2);
   if (steps == 0) return STH_OK;
+  if (ab.life_packed && steps >= kLifepMinSteps) {
+    if ((rc = iterate_life_packed(ctx, ab, ba, steps, flags, s))) return rc;
+    if (!(flags & STH_ASYNC)) STH_HIP(hipStreamSynchronize(s));
+    return STH_OK;
+  }
   // The first step runs the normalising kernel (it may read data this
   // library did not write); steps 1.. use the steady-state kernels.  With
   // graphs it is recorded at the head of the first graph launched.
@@ -1916,50 +2074,15 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
     for (int64_t i = 0; i < nplain && r2 == STH_OK; ++i) r2 = run_plan(i % 2 ? ab : ba, st, true);
     return r2;
   };
-  // Calls of a few launches go straight to the stream even with STH_GRAPH:
-  // a graph launch costs the host about 27 us against about 16 us for six
-  // direct launches, and the device is the bound either way (Life 8192^2,
-  // 20 steps: 152 us direct, 159 us replayed).
-  constexpr int64_t kGraphMinLaunches = 17;
   const int64_t launches = 1 + 2 * units + tail;
   if (!(flags & STH_GRAPH) || launches < kGraphMinLaunches) {
     if ((rc = enqueue(s, true, units, tail))) return rc;
   } else {
-    // Graphs of steady steps (starting from buffer b) are captured once per
-    // parameter set and replayed.  The lookup and the launches happen under
-    // ctx->mu, so a cache eviction on another thread cannot destroy an
-    // executable between the two.
     auto launch_graph = [&](const char* tag, bool first, int64_t nunits, int64_t nplain, int64_t times) -> int {
-      std::string key(reinterpret_cast<const char*>(&ab), sizeof(Plan));
-      key.append(reinterpret_cast<const char*>(&ba), sizeof(Plan));
-      key.append(tag);
-      key.push_back(first ? '1' : '0');
+      std::string key = std::string(tag) + (first ? '1' : '0');
       key.append(reinterpret_cast<const char*>(&nunits), sizeof nunits);
       key.append(reinterpret_cast<const char*>(&nplain), sizeof nplain);
-      std::lock_guard<std::mutex> lk(ctx->mu);
-      auto it = ctx->graphs.find(key);
-      if (it != ctx->graphs.end()) {
-        for (int64_t i = 0; i < times; ++i) STH_HIP(hipGraphLaunch(it->second, s));
-        return STH_OK;
-      }
-      STH_HIP(hipStreamBeginCapture(ctx->capture, hipStreamCaptureModeThreadLocal));
-      const int r2 = enqueue(ctx->capture, first, nunits, nplain);
-      hipGraph_t g = nullptr;
-      hipError_t e = hipStreamEndCapture(ctx->capture, &g);
-      if (r2) return r2;
-      if (e != hipSuccess) return fail(STH_EDEVICE, "hipStreamEndCapture: %s", hipGetErrorString(e));
-      hipGraphExec_t x = nullptr;
-      e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (e != hipSuccess) return fail(STH_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e));
-      if (ctx->graphs.size() >= kMaxGraphs) {
-        // bound the cache (a long-running caller iterating ever new buffers
-        // would grow it without end): wait for the device, then drop it all
-        if (int r3 = clear_graphs(ctx)) return r3;
-      }
-      ctx->graphs.emplace(key, x);
-      for (int64_t i = 0; i < times; ++i) STH_HIP(hipGraphLaunch(x, s));
-      return STH_OK;
+      return replay_graph(ctx, ab, ba, key, times, s, [&](hipStream_t st) { return enqueue(st, first, nunits, nplain); });
     };
     // the first graph launched carries the first step; a call's graphs
     // (head, repeated body, tail) are one graph when the call is short
