@@ -393,7 +393,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
     pl.life_packed = 1;
   const std::string bucket = "|c" + std::to_string(ilog2(cells)) + "|x" + std::to_string(ilog2(n[0]));
   if (!(flags & STH_GENERIC) && op->kind == STH_OP_LIFE && (sdt == STH_U8 || sdt == STH_BOOL) &&
-      moore1 && src->ndim == 2 && n[0] % 16 == 0 && aligned16(p.src) && aligned16(p.dst)) {
+      moore1 && src->ndim == 2 && n[0] >= 16 && n[0] < (int64_t(1) << 30) && n[1] < (int64_t(1) << 30)) {
     const bool conway = op->birth_mask == (1ull << 3) && op->survive_mask == ((1ull << 2) | (1ull << 3));
     // Every byte this kernel writes is 0 or 1, so later steps of an iteration
     // can skip normalising the source -- unless they read a halo (Use).
@@ -428,7 +428,8 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
     }
     // Conway's rule under Wrap / Remove / Reflect on grids below 2 GiB:
     // several generations per launch with one bit per cell (lifeb_kernel)
-    const bool bitlife = conway && (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= 16 &&
+    const bool vec16 = n[0] % 16 == 0 && aligned16(p.src) && aligned16(p.dst);  // both kernels' chunks
+    const bool bitlife = vec16 && conway && (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= 16 &&
                          zm2_extent(p.src, 1) < kZm2MaxBytes && zm2_extent(p.dst, 1) < kZm2MaxBytes;
     if (bc != STH_USE && n[1] >= 3 && bitlife) {
       // generations per launch (STH_LIFEB_G: 2, 4 or 8) and waves per launch
@@ -450,7 +451,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       pl.fused_gens = lg;
       lifeb_grid(n[0], n[1], lg, lwaves, &pl.fused_tiles_x, &pl.fused_tiles_y);
       pl.fused_tiles_z = 1;
-    } else if (bc != STH_USE && n[1] >= 3) {
+    } else if (vec16 && bc != STH_USE && n[1] >= 3) {
       // temporal blocking for steady iteration steps (two generations per launch)
       int ky2 = 8;  // rows per wave of the fused kernel (measured best; STH_LIFE2_KY: 2, 4 or 8)
       if (const char* e = std::getenv("STH_LIFE2_KY")) ky2 = std::atoi(e);
@@ -1302,6 +1303,7 @@ int iterate_life_packed(sth_ctx* ctx, const Plan& ab, const Plan& ba, int64_t st
   q.n0 = static_cast<int32_t>(m.src.n0);
   q.n1 = static_cast<int32_t>(m.src.n1);
   q.words = lifep_words(m.src.n0);
+  q.lpr_shift = shape.lpr_shift;
   q.pad = (m.padval & 0xffu) ? 0xffffffffu : 0u;
   q.birth = static_cast<uint32_t>(m.op.birth & 0x1ffu);
   q.survive = static_cast<uint32_t>(m.op.survive & 0x1ffu);
@@ -1322,7 +1324,7 @@ int iterate_life_packed(sth_ctx* ctx, const Plan& ab, const Plan& ba, int64_t st
   auto advance = [&](hipStream_t st, int64_t i, int64_t g) -> int {
     LifepParams l = between(i % 2 != 0);
     l.gens = static_cast<int32_t>(g);
-    lifep_grid(l.n0, l.n1, shape.k, l.gens, &l.tiles_x, &l.tiles_y);
+    lifep_grid(l.n0, l.n1, shape.k, l.gens, shape.lpr_shift, &l.tiles_x, &l.tiles_y);
     launch(l, st);
     STH_HIP(hipGetLastError());
     return STH_OK;

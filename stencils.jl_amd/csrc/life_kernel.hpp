@@ -17,13 +17,23 @@
 // update_boundary! does before the reference's kernel (src/array.jl:195-242):
 // no thread reads the halo during the step, so the writes cannot race.
 //
-// Preconditions checked on the host: 2-D, n0 % 16 == 0, interior rows of
-// source and destination 16-byte aligned.
+// Rows may start on any byte and hold any number of cells from 16 on: a
+// chunk is one 16-byte access at any address, and the last lane of a row
+// whose length is no multiple of 16 owns the row's last 16 cells (some of
+// them also its neighbour's, with the same results).  A grid of 1501 x 1333
+// cells took the runtime-offset tile kernel 13.6 us per generation before.
 #pragma once
 
 #include "common.hpp"
 
 namespace sth {
+
+// A lane's 16 cells at any address, one access.
+__device__ __forceinline__ uint4 life_load(const uint8_t* p) {
+  uint4 v;
+  __builtin_memcpy(&v, p, sizeof v);
+  return v;
+}
 
 // Cross-lane moves (DPP wave shifts, full rate): lane i receives lane i - 1
 // (from_left) or lane i + 1 (from_right); the lane with no such neighbour
@@ -90,7 +100,7 @@ __device__ __forceinline__ void life_rows(const MapParams& p, const uint8_t* __r
     for (int r = 0; r < NR; ++r) {
       padrow[r] = false;
       rowp[r] = row;
-      raw[r] = *reinterpret_cast<const uint4*>(row + xs);
+      raw[r] = life_load(row + xs);
       row += s1;
     }
   } else {
@@ -107,7 +117,7 @@ __device__ __forceinline__ void life_rows(const MapParams& p, const uint8_t* __r
       const int32_t ym = halo ? yc : (wrap ? yw : (refl ? yr : (out ? 0 : yc)));
       padrow[r] = !halo && !wrap && !refl && out;
       rowp[r] = src + static_cast<int64_t>(ym) * s1;
-      raw[r] = *reinterpret_cast<const uint4*>(rowp[r] + xs);
+      raw[r] = life_load(rowp[r] + xs);
     }
   }
   // The edge bytes (x0 - 1, x0 + 16) come from the neighbouring lanes'
@@ -184,7 +194,7 @@ __device__ __forceinline__ void life_rows(const MapParams& p, const uint8_t* __r
     for (int j = 0; j < KY; ++j) {
       if (EDGE && y0 + j >= n1) break;
       // (plain stores: nontemporal ones measured 45% slower on MI355X here)
-      *reinterpret_cast<uint4*>(d) = outs[j];
+      __builtin_memcpy(d, &outs[j], sizeof(uint4));
       d += p.dst.s1;
     }
   }
@@ -201,9 +211,11 @@ __global__ __launch_bounds__(256) void life_kernel(MapParams p) {
   const int brow = bid / p.tiles_x;
 
   const int32_t n0 = static_cast<int32_t>(p.src.n0), n1 = static_cast<int32_t>(p.src.n1);
-  const int32_t x0 = (bcol * 64 + lane) * 16;
+  const int32_t xc = (bcol * 64 + lane) * 16;
   const int32_t y0 = (brow * 4 + wave) * KY;
-  const bool active = x0 < n0;
+  const bool active = xc < n0;
+  const bool shifted = active && xc + 16 > n0;  // the row's last 16 cells
+  const int32_t x0 = shifted ? n0 - 16 : xc;
   const int bc = p.bc;
   const bool halo = p.read_halo != 0;
   const uint8_t* src = reinterpret_cast<const uint8_t*>(p.src.base);
@@ -220,10 +232,11 @@ __global__ __launch_bounds__(256) void life_kernel(MapParams p) {
   const int32_t xlm = halo ? xl : (lpad ? 0 : static_cast<int32_t>(map_index(xl, n0, bc)));
   const int32_t xrm = halo ? xr : (rpad ? 0 : static_cast<int32_t>(map_index(xr, n0, bc)));
 
-  // lanes whose neighbour chunk is outside this wave or the array load the
-  // edge byte themselves (every lane takes part in the cross-lane moves)
-  const bool fill_l = lane == 0 || xs == 0;
-  const bool fill_r = lane == 63 || xs + 16 >= n0 || x0 + 16 >= n0;
+  // lanes whose neighbour chunk is outside this wave or the array, or not
+  // the adjacent 16 cells, load the edge byte themselves (every lane takes
+  // part in the cross-lane moves)
+  const bool fill_l = lane == 0 || xs == 0 || shifted;
+  const bool fill_r = lane == 63 || xc + 32 > n0;
   if (y0 >= 1 && y0 + KY < n1)
     life_rows<KY, CONWAY, NORM, false>(p, src, dst, x0, y0, active, xs, xlm, xrm, lpad, rpad, fill_l, fill_r);
   else

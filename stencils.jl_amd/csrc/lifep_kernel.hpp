@@ -10,20 +10,23 @@
 // single steps that end every iteration.
 //
 // lifep_kernel: a lane holds one 32-cell word of K consecutive rows in
-// registers, a wave 64 words (2 rim words and 62 words of results) and a
-// workgroup 16 waves stacked along the rows.  Per generation each wave hands
-// its first and last row to its neighbours through LDS (two buffers, one
-// barrier) and computes its interior rows before it waits.  The tile's outer
+// registers.  `lpr` = 64, 32 or 16 lanes stand side by side (two of them rim
+// words, the others results) and the 64 / lpr groups of a wave one above the
+// other; a workgroup stacks 16 waves.  Per generation each group hands its
+// first and last row to its neighbours through LDS (two buffers, one
+// barrier); interior rows are computed before the wait.  The tile's outer
 // rows and the rim words lose one row / one bit per generation, so a launch
 // of `gens` generations stores the tile without `gens` rows on each side,
-// and gens <= 32 keeps all 62 words exact.
+// and gens <= 32 keeps the other words exact.
 //
-// Why this split: a generation of Conway's rule costs 14 full-rate VALU
-// operations per 32 cells (2 lane moves, 2 funnel shifts and 10 v_bitop3),
-// against 12 per 16 cells for windows that carry their own rim bits, and a
-// tile of 16 K rows recomputes only 2 gens rows where a wave marching alone
-// down a chunk of 32 rows recomputed 2 gens of every 32 + 2 gens.  Packed
-// rows move 1/8 of the bytes, so memory no longer bounds it.
+// Why this split: a generation of Conway's rule costs 15 full-rate VALU
+// operations per 32 cells (2 lane moves, 2 funnel shifts, 10 v_bitop3 and the
+// share of the exchanged rows), against 12 per 16 cells for windows that
+// carry their own rim bits, and a tile recomputes only its rim where a wave
+// marching alone down a chunk of 32 rows recomputed 2 gens of every
+// 32 + 2 gens.  Groups of 32 or 16 lanes make the tile squarer (less rim) and
+// fit more widths.  Packed rows move 1/8 of the bytes; the kernel is bound by
+// VALU issue, and by the load and store of the tile, which do not overlap.
 //
 // Cells outside the array follow the reference's getneighbor
 // (src/array.jl:129-179) in every generation: Wrap and Reflect load rows and
@@ -33,17 +36,17 @@
 // every generation.
 #pragma once
 
+#include <algorithm>
+
 #include "lifeb_kernel.hpp"
 
 namespace sth {
 
-// Packed row y of a buffer: 4-byte words from the first 4-byte boundary of
-// the row, in one of four slots by row: consecutive rows of a pitch of 2^k
-// bytes would otherwise start on the same memory channel and use 1/8 of
-// them.  n0 >= kLifepMinN0 leaves room for the slots inside every row.
+// Packed row y of a buffer: 4-byte words in the cells of row y / 4, which
+// holds four packed rows one after another from its first 4-byte boundary
+// on.  n0 >= kLifepMinN0 leaves room for them.
 constexpr int kLifepMinN0 = 64;
 constexpr int kLifepWaves = 16;   // waves of a workgroup
-constexpr int kLifepOut = 62;     // words of results per wave
 constexpr int kLifepMaxGens = 32; // a rim word's bits
 
 struct LifepParams {
@@ -53,6 +56,7 @@ struct LifepParams {
   int32_t n0, n1;
   int32_t words;   // packed words per row
   int32_t gens;    // generations of this launch
+  int32_t lpr_shift;  // log2 of the lanes side by side
   int32_t tiles_x, tiles_y;
   uint32_t pad;    // 0 or ~0: the padval's bit
   uint32_t birth, survive;  // neighbour counts 0..8
@@ -61,7 +65,7 @@ struct LifepParams {
 __host__ __device__ __forceinline__ int32_t lifep_words(int64_t n0) { return static_cast<int32_t>((n0 + 31) >> 5); }
 
 __device__ __forceinline__ uint32_t* lifep_row(char* base, int64_t pitch, int32_t y, int32_t words) {
-  const uint64_t a = (reinterpret_cast<uint64_t>(base + static_cast<int64_t>(y) * pitch) + 3) & ~uint64_t(3);
+  const uint64_t a = (reinterpret_cast<uint64_t>(base + static_cast<int64_t>(y >> 2) * pitch) + 3) & ~uint64_t(3);
   return reinterpret_cast<uint32_t*>(a) + (y & 3) * words;
 }
 
@@ -107,151 +111,176 @@ __device__ __forceinline__ uint32_t lifep_rule(uint32_t sa, uint32_t ca, uint32_
 template <int K, bool CONWAY, int BC>
 __global__ __launch_bounds__(kLifepWaves * 64) void lifep_kernel(LifepParams p) {
   constexpr bool REMOVE = BC == STH_REMOVE, REFLECT = BC == STH_REFLECT;
-  __shared__ uint32_t edge[2][kLifepWaves][2][64];  // first and last row of every wave, two generations
-  const int lane = static_cast<int>(threadIdx.x & 63);
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  __shared__ uint32_t edge[2][kLifepWaves * 2 * 64];  // first and last row of every group, two generations
+  const int lpr = 1 << p.lpr_shift, groups = kLifepWaves << (6 - p.lpr_shift);
+  const int col = static_cast<int>(threadIdx.x) & (lpr - 1);
+  const int group = static_cast<int>(threadIdx.x) >> p.lpr_shift;
   const int tile = xcd_block_id(static_cast<int>(blockIdx.x), p.tiles_x * p.tiles_y, 1);
   const int strip = tile % p.tiles_x;
   const int32_t n0 = p.n0, n1 = p.n1, words = p.words, gens = p.gens;
   // rows of the tile: gens rim rows, the results, gens rim rows
-  const int32_t y0 = (tile / p.tiles_x) * (kLifepWaves * K - 2 * gens) - gens + wave * K;
-  const int32_t wi = strip * kLifepOut - 1 + lane;  // this lane's word
-  const int32_t c = wi * 32;                        // its first column
-  // waves with a word that is not wholly inside the row (uniform)
-  const bool xedge = strip == 0 || (strip * kLifepOut + 63) * 32 > n0;
+  const int32_t t0 = (tile / p.tiles_x) * (groups * K - 2 * gens) - gens;
+  const int32_t y0 = t0 + group * K;             // this lane's first row
+  const int32_t wi = strip * (lpr - 2) - 1 + col;  // its word
+  const int32_t c = wi * 32;                     // the word's first column
+  // tiles with a word that is not wholly inside the row, or a row outside
+  const bool xedge = strip == 0 || (strip * (lpr - 2) + lpr - 1) * 32 > n0;
+  const bool yedge = t0 < 0 || t0 + groups * K > n1;
 
-  // ---- load
+  // ---- load: every load of the lane's rows is issued before the first use
   uint32_t w[K];
   uint32_t keep = 0xffffffffu;  // bits of columns inside the row
+  if (c < 0 || c >= n0) keep = 0u;
+  else if (c + 32 > n0) keep = (1u << (n0 - c)) - 1u;
   {
-    if (c < 0 || c >= n0) keep = 0u;
-    else if (c + 32 > n0) keep = (1u << (n0 - c)) - 1u;
-    // edge words: own bits from bit pa (masked), the rest from bit pb on,
-    // moved up by q (Wrap) or reversed (Reflect)
-    int32_t pa = 0, pb = 0, q = 0;
-    if constexpr (!REMOVE) {
-      pa = keep ? c : 0;
-      if (c < 0) {
-        pb = REFLECT ? 1 : n0 - 32;
-      } else if (c < n0) {
-        q = REFLECT ? 0 : (n0 - c) & 31;
-        pb = REFLECT ? 2 * n0 - 33 - c : 0;
-      } else {
-        pb = REFLECT ? 2 * n0 - 33 - c : c - n0;
-      }
-      if (pb < 0 || pb > n0) pb = 0;  // words too far out to reach a result
-    } else {
-      pa = keep ? c : 0;
-    }
+    const uint32_t* row[K];
 #pragma unroll
     for (int r = 0; r < K; ++r) {
-      const int32_t y = y0 + r;
-      const int32_t ym = REMOVE ? (y < 0 ? 0 : (y >= n1 ? n1 - 1 : y)) : lifeb_map_row(y, n1, REFLECT);
-      const uint32_t* row = lifep_row(p.src, p.s1, ym, words);
-      if (!xedge) {
-        w[r] = row[wi];
-      } else {
-        const uint32_t own = row[pa >> 5];
+      int32_t ym = y0 + r;
+      if (yedge) ym = REMOVE ? (ym < 0 ? 0 : (ym >= n1 ? n1 - 1 : ym)) : lifeb_map_row(ym, n1, REFLECT);
+      row[r] = lifep_row(p.src, p.s1, ym, words);
+    }
+    if (!xedge) {
+#pragma unroll
+      for (int r = 0; r < K; ++r) w[r] = row[r][wi];
+    } else {
+      // own bits (masked); the rest from bit pb on, moved up by q (Wrap) or
+      // reversed (Reflect), or padval
+      const int32_t io = keep ? wi : 0;
+      int32_t pb = 0, q = 0;
+      uint32_t lo[K], hi[K];
+      if constexpr (!REMOVE) {
+        if (c < 0) {
+          pb = REFLECT ? 1 : n0 - 32;
+        } else if (c < n0) {
+          q = REFLECT ? 0 : (n0 - c) & 31;
+          pb = REFLECT ? 2 * n0 - 33 - c : 0;
+        } else {
+          pb = REFLECT ? 2 * n0 - 33 - c : c - n0;
+        }
+        if (pb < 0 || pb > n0) pb = 0;  // words too far out to reach a result
+        const int32_t i = pb >> 5, i0 = i < words ? i : words - 1, i1 = i + 1 < words ? i + 1 : words - 1;
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+          lo[r] = row[r][i0];
+          hi[r] = row[r][i1];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < K; ++r) w[r] = row[r][io];
+#pragma unroll
+      for (int r = 0; r < K; ++r) {
         uint32_t far = p.pad;
         if constexpr (!REMOVE) {
-          far = lifep_bits(row, pb, words);
+          far = __builtin_amdgcn_alignbit(hi[r], lo[r], pb & 31);
           far = REFLECT ? __builtin_bitreverse32(far) : far << q;
         }
-        w[r] = (own & keep) | (far & ~keep);
-      }
-      if constexpr (REMOVE) {
-        if (y < 0 || y >= n1) w[r] = p.pad;
+        w[r] = (w[r] & keep) | (far & ~keep);
       }
     }
   }
-  // Remove: waves with outside rows or bits reset them every generation
-  const bool reset = REMOVE && (xedge || y0 < 0 || y0 + K > n1);
+  // Remove: tiles with outside rows or bits set them to padval, now and after
+  // every generation
+  const bool reset = REMOVE && (xedge || yedge);
+  auto held = [&](uint32_t v, int r) -> uint32_t {
+    const uint32_t k = y0 + r < 0 || y0 + r >= n1 ? 0u : keep;
+    return bop3<(kA3 & kB3) | (~kB3 & kC3)>(v, k, p.pad);
+  };
+  if (reset) {
+#pragma unroll
+    for (int r = 0; r < K; ++r) w[r] = held(w[r], r);
+  }
 
   // ---- generations
-  edge[0][wave][0][lane] = w[0];
-  edge[0][wave][1][lane] = w[K - 1];
+  uint32_t* const mine = &edge[0][(group * 2) * lpr + col];  // first row; last row lpr further
+  const uint32_t* const above = group > 0 ? mine - lpr : mine;
+  const uint32_t* const below = group < groups - 1 ? mine + 2 * lpr : mine;
+  constexpr int kBuf = kLifepWaves * 2 * 64;
+  mine[0] = w[0];
+  mine[lpr] = w[K - 1];
   for (int g = 0; g < gens; ++g) {
     uint32_t hs[K], hc[K];
 #pragma unroll
     for (int r = 0; r < K; ++r) lifep_hsum(w[r], hs[r], hc[r]);
     auto next = [&](uint32_t sa, uint32_t ca, int r, uint32_t sc, uint32_t cc) -> uint32_t {
-      uint32_t v;
-      if constexpr (CONWAY) v = conway_bits(sa, ca, hs[r], hc[r], sc, cc, w[r]);
-      else v = lifep_rule(sa, ca, hs[r], hc[r], sc, cc, w[r], p.birth, p.survive);
-      if constexpr (REMOVE) {
-        if (reset) {
-          const int32_t y = y0 + r;
-          v = bop3<(kA3 & kB3) | (~kB3 & kC3)>(v, keep, p.pad);
-          if (y < 0 || y >= n1) v = p.pad;
-        }
-      }
-      return v;
+      if constexpr (CONWAY) return conway_bits(sa, ca, hs[r], hc[r], sc, cc, w[r]);
+      else return lifep_rule(sa, ca, hs[r], hc[r], sc, cc, w[r], p.birth, p.survive);
     };
     uint32_t v[K];
 #pragma unroll
     for (int r = 1; r + 1 < K; ++r) v[r] = next(hs[r - 1], hc[r - 1], r, hs[r + 1], hc[r + 1]);
-    // the neighbours' rows of this generation (the outermost waves': any)
+    // the neighbours' rows of this generation (the outermost groups': any)
     __syncthreads();
-    const int b = g & 1;
+    const int b = (g & 1) * kBuf;
     uint32_t ts, tc, bs, bc;
-    lifep_hsum(edge[b][wave > 0 ? wave - 1 : 0][1][lane], ts, tc);
-    lifep_hsum(edge[b][wave < kLifepWaves - 1 ? wave + 1 : wave][0][lane], bs, bc);
+    lifep_hsum(above[b], ts, tc);
+    lifep_hsum(below[b], bs, bc);
     if constexpr (K == 1) {
       v[0] = next(ts, tc, 0, bs, bc);
     } else {
       v[0] = next(ts, tc, 0, hs[1], hc[1]);
       v[K - 1] = next(hs[K - 2], hc[K - 2], K - 1, bs, bc);
     }
+    if (reset) {
+#pragma unroll
+      for (int r = 0; r < K; ++r) v[r] = held(v[r], r);
+    }
 #pragma unroll
     for (int r = 0; r < K; ++r) w[r] = v[r];
-    edge[b ^ 1][wave][0][lane] = w[0];
-    edge[b ^ 1][wave][1][lane] = w[K - 1];
+    mine[kBuf - b] = w[0];
+    mine[kBuf - b + lpr] = w[K - 1];
   }
 
   // ---- store
-  if (lane >= 1 && lane <= kLifepOut && wi < words) {
+  if (col >= 1 && col <= lpr - 2 && wi < words) {
 #pragma unroll
     for (int r = 0; r < K; ++r) {
-      const int32_t l = wave * K + r, y = y0 + r;  // y >= 0 for every result row
-      if (l >= gens && l < kLifepWaves * K - gens && y < n1) lifep_row(p.dst, p.d1, y, words)[wi] = w[r];
+      const int32_t l = group * K + r, y = y0 + r;  // y >= 0 for every result row
+      if (l >= gens && l < groups * K - gens && y < n1) lifep_row(p.dst, p.d1, y, words)[wi] = w[r];
     }
   }
 }
 
 // ------------------------------------------------------------ host side
 
-// Rows per wave and generations per launch for an n0 x n1 grid: the pair
-// with the least time per generation by a model in cycles of one SIMD -- a
-// tile's 4 waves per SIMD take 4 cycles per operation and row, every tile a
-// CU runs adds to that, a generation's exchange costs about 350 and a launch
-// (its start, loads and stores) about 6000.
+// Rows per lane, generations per launch and lanes side by side for an
+// n0 x n1 grid: those with the least time per generation by a model fitted to measured launches
+// (in microseconds, 64 lanes side by side; 8192^2: K = 12, G = 1 / 8 / 15 take 9.4 / 16.7 / 23.6,
+// K = 6, G = 7 takes 14.5; 4096^2: K = 6, G = 16 / 23 take 14.8 / 19.0;
+// 1501 x 1333: K = 1, G = 4 takes 3.9, K = 3, G = 8 / 16 take 6.4 / 9.3).  A
+// launch costs 2.7 and 0.7 per MB of packed grid (its loads and stores are
+// not overlapped with generations); a generation costs 0.083 per row of a
+// wave and tile a CU holds, and at least its exchange, 0.25 + 0.05 K.
 struct LifepShape {
-  int32_t k, gens, tiles_x, tiles_y;
+  int32_t k, gens, lpr_shift;
 };
-constexpr int kLifepRows[] = {1, 2, 3, 4, 6, 8, 10, 12, 14, 16};
+constexpr int kLifepRows[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 14, 16};
 
-inline void lifep_grid(int64_t n0, int64_t n1, int k, int gens, int32_t* tx, int32_t* ty) {
-  *tx = static_cast<int32_t>((lifep_words(n0) + kLifepOut - 1) / kLifepOut);
-  const int64_t rows = kLifepWaves * k - 2 * gens;
+inline void lifep_grid(int64_t n0, int64_t n1, int k, int gens, int lpr_shift, int32_t* tx, int32_t* ty) {
+  const int out = (1 << lpr_shift) - 2;
+  *tx = static_cast<int32_t>((lifep_words(n0) + out - 1) / out);
+  const int64_t rows = (kLifepWaves << (6 - lpr_shift)) * k - 2 * gens;
   *ty = static_cast<int32_t>((n1 + rows - 1) / rows);
 }
 
 inline LifepShape lifep_shape(int64_t n0, int64_t n1, bool conway, int cus) {
   LifepShape best{};
   double least = 0;
-  const double ops = conway ? 14 : 38;
-  for (int k : kLifepRows)
-    for (int g = 2; g <= kLifepMaxGens && kLifepWaves * k - 2 * g >= 1; ++g) {
-      LifepShape s{k, g, 0, 0};
-      lifep_grid(n0, n1, k, g, &s.tiles_x, &s.tiles_y);
-      const int64_t tiles = static_cast<int64_t>(s.tiles_x) * s.tiles_y;
-      const double rounds = static_cast<double>((tiles + cus - 1) / cus);
-      const double t = 6000.0 / g + 350.0 + rounds * (kLifepWaves / 4) * 4.0 * k * ops;
-      if (!best.k || t < least) {
-        best = s;
-        least = t;
+  const double work = conway ? 1.0 : 2.6;  // operations per word against Conway's 15
+  const double fixed = 2.7 + 0.7e-6 * (static_cast<double>(n0) * static_cast<double>(n1) / 8.0);
+  for (int sh = 4; sh <= 6; ++sh)
+    for (int k : kLifepRows)
+      for (int g = 2; g <= kLifepMaxGens && (kLifepWaves << (6 - sh)) * k - 2 * g >= 1; ++g) {
+        int32_t tx, ty;
+        lifep_grid(n0, n1, k, g, sh, &tx, &ty);
+        const int64_t tiles = static_cast<int64_t>(tx) * ty;
+        const double per_cu = static_cast<double>((tiles + cus - 1) / cus);
+        const double t = fixed / g + std::max(0.25 + 0.05 * k * work, 0.08 + per_cu * 0.083 * k * work);
+        if (!best.k || t < least) {
+          best = LifepShape{k, g, sh};
+          least = t;
+        }
       }
-    }
   return best;
 }
 

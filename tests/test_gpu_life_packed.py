@@ -37,6 +37,30 @@ def test_packed_life_iterations(gpu, oracle, shape, bname):
         np.testing.assert_array_equal(G.dest, O.dest, err_msg=msg)
 
 
+@pytest.mark.parametrize("bname", ["remove1", "wrap", "reflect", "use"])
+@pytest.mark.parametrize("shape", [(18, 9), (33, 5), (63, 34), (1025, 7), (1039, 33)])
+def test_single_steps_on_rows_of_any_length(gpu, oracle, shape, bname):
+    """Rows that are no multiple of 16 cells: the last lane's chunk overlaps
+    its neighbour's (csrc/life_kernel.hpp), every rows-per-lane variant."""
+    from stencils_hip import _lib
+    rng = np.random.default_rng(shape[0] + shape[1])
+    A = np.where(rng.random(shape) < 0.4, rng.integers(1, 256, shape), 0).astype(np.uint8)
+    bc = sh.Use() if bname == "use" else BOUNDS[bname]
+    for rule in (sh.LifeRule(), sh.LifeRule((1, 3, 6), (2, 3, 5))):
+        for pad in ("halo_in",) if bname == "use" else PADS:
+            make = lambda: sh.SwitchingStencilArray(A.copy(order="F"), sh.Moore(1), boundary=bc,  # noqa: E731
+                                                    padding=PADS[pad])
+            O = oracle.mapstencil_steps(rule, make(), 3)
+            for ky in ("ky2", "ky4", "ky8", "ky16"):
+                _lib.set_variant(ky)
+                try:
+                    G = sh.mapstencil_steps(rule, make(), 3)
+                finally:
+                    _lib.set_variant("")
+                np.testing.assert_array_equal(G.source, O.source, err_msg=f"{rule!r} {pad} {ky}")
+                np.testing.assert_array_equal(G.dest, O.dest, err_msg=f"{rule!r} {pad} {ky}")
+
+
 def test_packed_life_rows_of_a_view(gpu, oracle):
     """A grid inside a larger device tensor: rows start on any byte, and the
     cells between the rows are not the iteration's to write."""
