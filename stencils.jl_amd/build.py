@@ -123,7 +123,7 @@ def gen_static_tu(st, ops, ctype: str, code: str) -> str:
         '#include "stream_kernel.hpp"',
         '#include "zmarch2_kernel.hpp"',
         '#include "zmarch1_kernel.hpp"',
-        '#include "ymarch2_kernel.hpp"',
+        '#include "ymarch_kernel.hpp"',
         "namespace sth {",
         "namespace {",
         f"struct Shape_{name} {{",
@@ -164,11 +164,11 @@ def gen_static_tu(st, ops, ctype: str, code: str) -> str:
                 f"zmarch2_rows<Staged<{ctype}>::type>()}});")
             i += 1
         if st.N == 2 and max(rx, ry) <= 1:
-            # two steps per launch for iterations (2-D: march along y)
+            # several steps per launch for iterations (2-D: march along y)
             lines.append(
                 f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
-                f"&Shape_{name}::off[0][0], &launch_ymarch2<{ctype}, {op}, Shape_{name}>, "
-                f"ymarch2_v<Elem<{ctype}>::raw>()}});")
+                f"&Shape_{name}::off[0][0], &launch_ymarch<{ctype}, {op}, Shape_{name}>, "
+                f"ymarch_gens<Elem<{ctype}>::raw>({L})}});")
             i += 1
     lines += ["}  // namespace", "}  // namespace sth", ""]
     return "\n".join(lines)
@@ -263,7 +263,7 @@ def gen_runtime_tu(ctype: str) -> str:
 # library's own, minus host-only and include flags.
 JIT_HEADERS = [("stencils_hip.h", REPO / "include" / "stencils_hip.h"), ("common.hpp", CSRC / "common.hpp"),
                ("tile_kernel.hpp", CSRC / "tile_kernel.hpp"), ("stream_kernel.hpp", CSRC / "stream_kernel.hpp"),
-               ("zmarch2_kernel.hpp", CSRC / "zmarch2_kernel.hpp"), ("ymarch2_kernel.hpp", CSRC / "ymarch2_kernel.hpp"),
+               ("zmarch2_kernel.hpp", CSRC / "zmarch2_kernel.hpp"), ("ymarch_kernel.hpp", CSRC / "ymarch_kernel.hpp"),
                ("scatter_kernel.hpp", CSRC / "scatter_kernel.hpp")]
 JIT_OPTIONS = [f for f in CXXFLAGS if f not in ("-fPIC", "-Wno-unused-command-line-argument") and not f.startswith("-I")]
 

@@ -20,7 +20,7 @@
 #include "jit.hpp"
 #include "zmarch2_kernel.hpp"
 #include "zmarch1_kernel.hpp"
-#include "ymarch2_kernel.hpp"
+#include "ymarch_kernel.hpp"
 #include "life2_kernel.hpp"
 #include "lifeb_kernel.hpp"
 #include "life_kernel.hpp"
@@ -150,6 +150,7 @@ struct Plan {
   hipFunction_t jit_fused; // a runtime-compiled two-step kernel instead of fn_fused
   int32_t jit_fused_3d;    // its grid: tiles_x * tiles_y (2-D) or * tiles_z (3-D)
   int32_t fused_gens;      // steps fn_fused advances per launch
+  int32_t fused_any;       // it also advances any smaller number (MapParams::gens)
   int32_t fused_tiles_x, fused_tiles_y, fused_tiles_z;  // its grid
   int32_t life_packed;      // iterations may run on packed bits (lifep_kernel.hpp)
   HaloParams hp;
@@ -239,6 +240,9 @@ bool offsets_equal(const int8_t* tbl, int L, const std::vector<int>& offs3) {
       if (tbl[3 * k + d] != offs3[3 * k + d]) return false;
   return true;
 }
+
+// Compute units of an MI355X: what the marching kernels' grids are cut for.
+constexpr int kCus = 256;
 
 // Bytes from an array descriptor's base to the end of its last cell.
 int64_t zm2_extent(const DevArr& a, int64_t esize) {
@@ -637,33 +641,28 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
     }
   }
 
-  // two steps per launch for 2-D radius-1 catalogue stencils (Wrap / Remove /
-  // Reflect)
-  // on arrays whose rows start on 16-byte boundaries (the y-marching kernel
-  // loads whole vectors) and of 2^21 cells or more: 1.3-1.7x faster per step
-  // from 4096^2, mixed (0.6-1.3x) at 1024^2 (STH_FUSE2D_MIN_CELLS overrides)
+  // several steps per launch for 2-D radius-1 stencils (Wrap / Remove /
+  // Reflect) on arrays whose rows start on 4-byte boundaries (vectors are
+  // 16-byte buffer accesses at any such offset), of any size: 64^2 f32 heat
+  // takes 1.4 us per step against 2.7 with one launch per step
+  // (STH_FUSE2D_MIN_CELLS sets a smallest size)
   static const int64_t fuse2d_min = [] {
     const char* e = std::getenv("STH_FUSE2D_MIN_CELLS");
-    return e ? std::atoll(e) : (int64_t(1) << 21);
+    return e ? std::atoll(e) : int64_t(0);
   }();
-  auto rows16 = [](const DevArr& a, int64_t es) {
-    return reinterpret_cast<uintptr_t>(a.base) % 16 == 0 && (a.s1 * es) % 16 == 0;
+  auto rows4 = [](const DevArr& a, int64_t es) {
+    return reinterpret_cast<uintptr_t>(a.base) % 4 == 0 && (a.s1 * es) % 4 == 0;
   };
   if (!pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 2 && st->ndim == 2 &&
-      (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= 3 && n[1] >= 3 &&
+      (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= kYmMinCells && n[1] >= kYmMinCells &&
       n[0] * n[1] >= fuse2d_min &&
-      sdt == odt && rows16(pl.p.src, dtype_size(sdt)) && rows16(pl.p.dst, dtype_size(odt)) &&
+      sdt == odt && rows4(pl.p.src, dtype_size(sdt)) && rows4(pl.p.dst, dtype_size(odt)) &&
       zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes && zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes) {
     for (const auto& e : fused2_registry()) {
       if (e.dtype != sdt || e.op != op->kind || e.L != L || e.ndim != 2) continue;
       if (!offsets_equal(e.offs, L, offs3)) continue;
-      static const int64_t ym_waves = [] {
-        const char* v = std::getenv("STH_YM2_WAVES");
-        return v ? std::max<int64_t>(1, std::atoll(v)) : int64_t(8192);
-      }();
       pl.fn_fused = e.fn;
-      pl.fused_gens = 2;
-      ymarch2_grid(n[0], n[1], e.rows, ym_waves, &pl.fused_tiles_x, &pl.fused_tiles_y, &pl.fused_tiles_z);
+      pl.fused_gens = e.rows;
       break;
     }
     if (!pl.fn_fused && dtype_size(sdt) >= 2 && reach[0] <= 1 && reach[1] <= 1 && op->kind != STH_OP_LIFE &&
@@ -672,16 +671,17 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       for (size_t i = 0; i < o8.size(); ++i) o8[i] = static_cast<int8_t>(offs3[i]);
       std::string why;
       if (const JitKernel* jk = jit_fused_kernel(sdt, op->kind, L, o8.data(), 1, 1, 0, 2, bc, &why)) {
-        const char* v = std::getenv("STH_YM2_WAVES");
-        const int64_t yw = v ? std::max<int64_t>(1, std::atoll(v)) : int64_t(8192);
         pl.jit_fused = jk->fn;
         pl.jit_fused_3d = 0;
-        pl.fused_gens = 2;
-        ymarch2_grid(n[0], n[1], 16 / dtype_size(sdt), yw, &pl.fused_tiles_x, &pl.fused_tiles_y,
-                     &pl.fused_tiles_z);
+        pl.fused_gens = jit_ymarch_gens(sdt, L);
       } else {
-        jit_note("two-step 2-D kernel", why);
+        jit_note("multi-step 2-D kernel", why);
       }
+    }
+    if (pl.fn_fused || pl.jit_fused) {
+      pl.fused_any = 1;
+      ymarch_grid(n[0], n[1], 16 / dtype_size(sdt), pl.fused_gens, kCus, &pl.fused_tiles_x, &pl.fused_tiles_y,
+                  &pl.fused_tiles_z);
     }
   }
 
@@ -740,15 +740,18 @@ int run_plan(const Plan& pl, hipStream_t s, bool steady = false) {
   return STH_OK;
 }
 
-// Several steps in one launch (pl.fn_fused, steady state).  The fused kernels
-// map every boundary themselves and write only the destination's interior.
-int run_fused(const Plan& pl, hipStream_t s) {
+// Several steps in one launch (pl.fn_fused, steady state): pl.fused_gens, or
+// any smaller number `gens` where the kernel takes it (pl.fused_any).  The
+// fused kernels map every boundary themselves and write only the
+// destination's interior.
+int run_fused(const Plan& pl, hipStream_t s, int64_t gens = 0) {
   MapParams q = pl.p;
   q.tiles_x = pl.fused_tiles_x;
   q.tiles_y = pl.fused_tiles_y;
   q.tiles_z = pl.fused_tiles_z;
   q.read_halo = 0;
   q.fuse_halo = 0;
+  q.gens = gens ? static_cast<int32_t>(gens) : pl.fused_gens;
   if (pl.jit_fused) {
     const unsigned nb = static_cast<unsigned>(q.tiles_x) * q.tiles_y * (pl.jit_fused_3d ? q.tiles_z : 1);
     void* args[] = {&q};
@@ -1283,17 +1286,60 @@ int replay_graph(sth_ctx* ctx, const Plan& ab, const Plan& ba, const std::string
   return STH_OK;
 }
 
+// `gens` steps as launches of at most G steps each, the smallest number F of
+// launches that has the parity of `gens` (so the buffers alternate as step by
+// step): all take G steps but the last four, which share the rest.  Calls
+// head(stream), advance(stream, i, steps of launch i) and finish(stream, F);
+// with STH_GRAPH and enough launches 32 full launches are one graph,
+// replayed, and the rest of the call another (`kind` names the caller).
+template <class Head, class Advance, class Finish>
+int run_launches(sth_ctx* ctx, const Plan& ab, const Plan& ba, const char* kind, int64_t gens, int64_t G, uint32_t flags,
+                 hipStream_t s, Head&& head, Advance&& advance, Finish&& finish) {
+  int64_t F = (gens + G - 1) / G;
+  if ((F ^ gens) & 1) ++F;
+  const int64_t full = std::max<int64_t>(0, F - 4);
+  auto rest = [&](hipStream_t st, int64_t from) -> int {
+    int64_t left = gens - from * G;
+    for (int64_t i = from; i < F; ++i) {
+      const int64_t g = i < full ? G : (left + (F - i) - 1) / (F - i);
+      left -= g;
+      if (int rc = advance(st, i, g)) return rc;
+    }
+    return finish(st, F);
+  };
+  if (!(flags & STH_GRAPH) || F + 4 < kGraphMinLaunches) {
+    if (int rc = head(s)) return rc;
+    return rest(s, 0);
+  }
+  constexpr int64_t FU = 32;
+  const int64_t reps = full / FU;
+  auto tag = [&](char part, int64_t x) { return std::string(kind) + part + std::to_string(x); };
+  if (reps == 0)
+    return replay_graph(ctx, ab, ba, tag('a', gens), 1, s, [&](hipStream_t st) -> int {
+      const int rc = head(st);
+      return rc ? rc : rest(st, 0);
+    });
+  if (int rc = head(s)) return rc;
+  if (int rc = replay_graph(ctx, ab, ba, tag('b', G), reps, s, [&](hipStream_t st) -> int {
+        for (int64_t i = 0; i < FU; ++i)
+          if (int r2 = advance(st, i, G)) return r2;
+        return STH_OK;
+      }))
+    return rc;
+  return replay_graph(ctx, ab, ba, tag('r', gens - reps * FU * G), 1, s,
+                      [&](hipStream_t st) { return rest(st, reps * FU); });
+}
+
 // Fewest steps of a Life iteration that run packed: pack, launches in pairs,
 // unpack and two single steps are then no more launches than the steps.
 constexpr int64_t kLifepMinSteps = 8;
 
 // A Life iteration of `steps` generations from the a -> b plan `ab` and the
 // b -> a plan `ba`, on packed bits (lifep_kernel.hpp): a's cells are packed
-// into b, F launches advance steps - 2 generations between the buffers, the
+// into b, launches advance steps - 2 generations between the buffers, the
 // result is unpacked into the other buffer, and two single steps leave both
-// buffers and their halos as the step-by-step reference does.  F has the
-// parity of steps - 2, so those steps write the buffers they would write
-// step by step.  Every cell is 0 or 1 after the unpacking, as after a step.
+// buffers and their halos as the step-by-step reference does.  Every cell is
+// 0 or 1 after the unpacking, as after a step.
 int iterate_life_packed(sth_ctx* ctx, const Plan& ab, const Plan& ba, int64_t steps, uint32_t flags, hipStream_t s) {
   const MapParams& m = ab.p;
   const bool conway = m.op.birth == (1ull << 3) && m.op.survive == ((1ull << 2) | (1ull << 3));
@@ -1315,66 +1361,29 @@ int iterate_life_packed(sth_ctx* ctx, const Plan& ab, const Plan& ba, int64_t st
     q.d1 = y.s1;
     return q;
   };
-  const int64_t gens = steps - 2, G = shape.gens;
-  int64_t F = (gens + G - 1) / G;
-  if ((F ^ gens) & 1) ++F;
-  // all launches but the last four take G generations, those four share the rest
-  const int64_t full = std::max<int64_t>(0, F - 4);
   // launch i runs from b when i is even
-  auto advance = [&](hipStream_t st, int64_t i, int64_t g) -> int {
-    LifepParams l = between(i % 2 != 0);
-    l.gens = static_cast<int32_t>(g);
-    lifep_grid(l.n0, l.n1, shape.k, l.gens, shape.lpr_shift, &l.tiles_x, &l.tiles_y);
-    launch(l, st);
-    STH_HIP(hipGetLastError());
-    return STH_OK;
-  };
-  auto head = [&](hipStream_t st) -> int {
-    launch_life_pack(between(true), st);
-    STH_HIP(hipGetLastError());
-    return STH_OK;
-  };
-  auto tail = [&](hipStream_t st, int64_t from) -> int {
-    int r2 = STH_OK;
-    int64_t left = gens - from * G;
-    for (int64_t i = from; i < F && r2 == STH_OK; ++i) {
-      const int64_t g = i < full ? G : (left + (F - i) - 1) / (F - i);
-      left -= g;
-      r2 = advance(st, i, g);
-    }
-    if (r2) return r2;
-    launch_life_unpack(between(F % 2 != 0), st);
-    STH_HIP(hipGetLastError());
-    const Plan &p0 = F % 2 ? ba : ab, &p1 = F % 2 ? ab : ba;
-    if ((r2 = run_plan(p0, st, true))) return r2;
-    return run_plan(p1, st, true);
-  };
-  int rc;
-  const int64_t launches = F + 4;
-  if (!(flags & STH_GRAPH) || launches < kGraphMinLaunches) {
-    if ((rc = head(s))) return rc;
-    return tail(s, 0);
-  }
-  // graphs: 32 full launches (replayed), then the rest of the call
-  constexpr int64_t FU = 32;
-  const int64_t reps = full / FU;
-  auto tag = [](const char* t, int64_t x, int64_t y) {
-    return std::string(t) + std::to_string(x) + "," + std::to_string(y);
-  };
-  if (reps == 0)
-    return replay_graph(ctx, ab, ba, tag("lh", gens, 0), 1, s, [&](hipStream_t st) -> int {
-      const int r2 = head(st);
-      return r2 ? r2 : tail(st, 0);
-    });
-  if ((rc = head(s))) return rc;
-  if ((rc = replay_graph(ctx, ab, ba, tag("lb", G, FU), reps, s, [&](hipStream_t st) -> int {
-         int r2 = STH_OK;
-         for (int64_t i = 0; i < FU && r2 == STH_OK; ++i) r2 = advance(st, i, G);
-         return r2;
-       })))
-    return rc;
-  return replay_graph(ctx, ab, ba, tag("lt", gens - reps * FU * G, F - reps * FU), 1, s,
-                      [&](hipStream_t st) { return tail(st, reps * FU); });
+  return run_launches(
+      ctx, ab, ba, "life", steps - 2, shape.gens, flags, s,
+      [&](hipStream_t st) -> int {
+        launch_life_pack(between(true), st);
+        STH_HIP(hipGetLastError());
+        return STH_OK;
+      },
+      [&](hipStream_t st, int64_t i, int64_t g) -> int {
+        LifepParams l = between(i % 2 != 0);
+        l.gens = static_cast<int32_t>(g);
+        lifep_grid(l.n0, l.n1, shape.k, l.gens, shape.lpr_shift, &l.tiles_x, &l.tiles_y);
+        launch(l, st);
+        STH_HIP(hipGetLastError());
+        return STH_OK;
+      },
+      [&](hipStream_t st, int64_t F) -> int {
+        launch_life_unpack(between(F % 2 != 0), st);
+        STH_HIP(hipGetLastError());
+        const Plan &p0 = F % 2 ? ba : ab, &p1 = F % 2 ? ab : ba;
+        if (int rc = run_plan(p0, st, true)) return rc;
+        return run_plan(p1, st, true);
+      });
 }
 
 }  // namespace
@@ -2051,6 +2060,26 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
     if (!(flags & STH_ASYNC)) STH_HIP(hipStreamSynchronize(s));
     return STH_OK;
   }
+  if (ab.fused_any && ba.fused_any) {
+    // Several steps per launch, any number of them: the launches write only
+    // interiors and the newest generation, so the last step is a single one
+    // (the other buffer then holds the step before), and with a halo the
+    // last two (each refreshes its source's halo).
+    const int64_t single = ab.halo ? 2 : 1, gens = steps - single;
+    if (gens > 0 && (gens + ab.fused_gens - 1) / ab.fused_gens + 1 + single < steps) {
+      if ((rc = run_launches(
+               ctx, ab, ba, "flex", gens, ab.fused_gens, flags, s, [](hipStream_t) { return STH_OK; },
+               [&](hipStream_t st, int64_t i, int64_t g) { return run_fused(i % 2 ? ba : ab, st, g); },
+               [&](hipStream_t st, int64_t F) -> int {
+                 for (int64_t i = 0; i < single; ++i)
+                   if (int r2 = run_plan((F + i) % 2 ? ba : ab, st, true)) return r2;
+                 return STH_OK;
+               })))
+        return rc;
+      if (!(flags & STH_ASYNC)) STH_HIP(hipStreamSynchronize(s));
+      return STH_OK;
+    }
+  }
   // The first step runs the normalising kernel (it may read data this
   // library did not write); steps 1.. use the steady-state kernels.  With
   // graphs it is recorded at the head of the first graph launched.
@@ -2064,7 +2093,7 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
   // step-by-step reference does.
   const int64_t G = ab.fused_gens;
   const bool fuse = !(flags & STH_NO_FUSE) && (ab.fn_fused || ab.jit_fused) && (ba.fn_fused || ba.jit_fused) &&
-                    G >= 2 && rest >= 2 * G + 2;
+                    !ab.fused_any && !ba.fused_any && G >= 2 && rest >= 2 * G + 2;
   const int64_t units = fuse ? (rest - 2) / (2 * G) : 0;  // fused pairs
   const int64_t tail = rest - 2 * G * units;              // single steps (2 .. 2G + 1 when fused)
   auto enqueue = [&](hipStream_t st, bool first, int64_t nunits, int64_t nplain) -> int {

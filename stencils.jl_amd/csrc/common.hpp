@@ -23,7 +23,7 @@ __device__ __forceinline__ float bf16_to_float(uint16_t b) {
 // Round-to-nearest-even f32 -> bf16; NaN stays NaN (quiet bit forced): one
 // v_cvt_pk_bf16_f32, whose result equals the integer formulation
 // (x + 0x7fff + lsb) >> 16 for every one of the 2^32 inputs.  Six VALU
-// operations less per cell: bf16 Gaussian 5 x 5, 16384^2, 556 -> 517 us.
+// operations less per cell: bf16 Gaussian 7 x 7, 16384^2, 556 -> 517 us.
 __device__ __forceinline__ uint16_t float_to_bf16(float f) {
   return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
@@ -36,6 +36,25 @@ __device__ __forceinline__ float f16_to_float(uint16_t h) {
 #ifndef STH_OPAQUE
 #define STH_OPAQUE(x) __asm__("" : "+v"(x))
 #endif
+
+// A copy of a 4- or 8-byte value in other registers, made here (a move the
+// compiler cannot fold into renaming); other sizes pass through.
+template <typename T>
+__device__ __forceinline__ T copy_here(T v) {
+#ifndef STH_NO_ASM
+  if constexpr (sizeof(T) == 4) {
+    const uint32_t a = __builtin_bit_cast(uint32_t, v);
+    uint32_t r;
+    __asm__ volatile("v_mov_b32 %0, %1" : "=&v"(r) : "v"(a));
+    return __builtin_bit_cast(T, r);
+  } else if constexpr (sizeof(T) == 8) {
+    const uint64_t a = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = copy_here(static_cast<uint32_t>(a)), hi = copy_here(static_cast<uint32_t>(a >> 32));
+    return __builtin_bit_cast(T, (static_cast<uint64_t>(hi) << 32) | lo);
+  }
+#endif
+  return v;
+}
 
 __device__ __forceinline__ uint16_t float_to_f16(float f) {
   // Without the barrier the compiler folds the conversion into the producing
@@ -199,6 +218,8 @@ struct MapParams {
   int32_t fuse_halo;                  // Life kernel: read the interior only and refresh the
                                       // source halo in the same launch (update_boundary!)
   int32_t lpr_shift;                  // streaming kernels: log2 of the lanes per row (3..6)
+  int32_t gens;                       // y-marching kernel: steps of this launch
+  int32_t pad_;
   // runtime stencils: packed (dx, dy, dz) as int8 each in the low 24 bits
   int32_t offs[kMaxRuntimeL];
   // Kernel weights in the accumulator type (f64 uses both halves).

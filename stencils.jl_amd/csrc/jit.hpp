@@ -567,8 +567,15 @@ inline int jit_zmarch2_rows(int dtype) {
   return wide ? 10 : 16;
 }
 
-// The source of a two-step kernel (temporal blocking) specialised to one
-// radius-1 shape: ymarch2_kernel (2-D) or zmarch2_kernel (3-D) for
+// Most steps per launch of the 2-D multi-step kernel for storage type
+// `dtype`, as ymarch_gens gives it on the device.
+inline int jit_ymarch_gens(int dtype, int L) {
+  const bool half = dtype == STH_BF16 || dtype == STH_F16 || dtype == STH_I16 || dtype == STH_U16;
+  return half ? 4 : (L <= 4 ? 8 : 6);
+}
+
+// The source of a multi-step kernel (temporal blocking) specialised to one
+// radius-1 shape: ymarch_kernel (2-D) or zmarch2_kernel (3-D) for
 // boundary `bc` (false: no type name).
 inline bool jit_fused_source(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz, int ndim, int bc,
                              std::string* src_out, std::string* expr_out) {
@@ -576,9 +583,9 @@ inline bool jit_fused_source(int dtype, int opk, int L, const int8_t* offs3, int
   if (!tn) return false;
   const std::string head = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, ";
   const std::string targs = ndim == 3 ? head + std::to_string(jit_zmarch2_rows(dtype)) + ", " + std::to_string(bc)
-                                      : head + std::to_string(bc);
-  const std::string kern = ndim == 3 ? "zmarch2_kernel" : "ymarch2_kernel";
-  *src_out = "#include \"ymarch2_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, rz) +
+                                      : head + std::to_string(jit_ymarch_gens(dtype, L)) + ", " + std::to_string(bc);
+  const std::string kern = ndim == 3 ? "zmarch2_kernel" : "ymarch_kernel";
+  *src_out = "#include \"ymarch_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, rz) +
              "namespace sth {\ntemplate __global__ void " + kern + "<" + targs + ">(MapParams);\n}  // namespace sth\n";
   *expr_out = "&sth::" + kern + "<" + targs + ">";
   return true;
@@ -591,7 +598,7 @@ inline const JitKernel* jit_fused_kernel(int dtype, int opk, int L, const int8_t
     *why = "no type name";
     return nullptr;
   }
-  return jit_load(src, expr, ndim == 3 ? "zmarch2" : "ymarch2", why);
+  return jit_load(src, expr, ndim == 3 ? "zmarch2" : "ymarch", why);
 }
 
 // The scatter kernel with the interior order of each dest-column residue as

@@ -52,7 +52,7 @@ struct KernelEntry {
 
 std::vector<KernelEntry>& registry();
 
-// Kernels that advance an iteration by two steps per launch (temporal
+// Kernels that advance an iteration by several steps per launch (temporal
 // blocking), matched like KernelEntry.
 struct Fused2Entry {
   int dtype;
@@ -61,7 +61,7 @@ struct Fused2Entry {
   int ndim;
   const int8_t* offs;
   LaunchFn fn;
-  int rows;  // 3-D: rows per wave of the z-marching kernel; 2-D: cells per lane
+  int rows;  // 3-D (two steps): rows per wave of the z-marching kernel; 2-D: most steps per launch
 };
 std::vector<Fused2Entry>& fused2_registry();
 

@@ -15,9 +15,9 @@
 //                 step is one batched launch over the active requests
 //                 (requests join and leave only between rounds), buffers
 //                 ping-pong per request.  Requests of 2^21 cells or more
-//                 that have a two-step kernel run their own launches
-//                 instead, two steps each, up to 4 x round_steps steps per
-//                 round.  Requests that reach their step count get
+//                 that have a multi-step kernel run their own launches
+//                 instead, several steps each, up to 4 x round_steps steps
+//                 per round.  Requests that reach their step count get
 //                 their state copied to `result` and an event recorded.
 // Launches are stream-ordered, so a freed buffer is reused only by work
 // enqueued after the copy that last read it.  The host runs at most two
@@ -267,10 +267,10 @@ struct sth_server {
   }
 
   // --- 3. one round (called without `mu`: only the scheduler touches `active`)
-  // A request with a two-step kernel (3-D and 2-D radius-1 stencils, Life)
+  // A request with a multi-step kernel (3-D and 2-D radius-1 stencils, Life)
   // and at least 2^21 cells runs as
-  // launches of its own: two steps per launch, and more steps per round than
-  // the shared batch.  Below that size batching the steps pays more.
+  // launches of its own: several steps per launch, and more steps per round
+  // than the shared batch.  Below that size batching the steps pays more.
   // (STH_SERVER_SOLO_CELLS overrides the size)
   static int64_t solo_cells() {
     static const int64_t v = [] {
@@ -292,7 +292,7 @@ struct sth_server {
   int advance_solo(Req& q, int64_t n, int64_t* launches) {
     const hipStream_t st = solo_streams[q.lane];
     if (q.done == 0 && n > 0) {
-      // the first step is a single step, as in sth_iterate: the two-step
+      // the first step is a single step, as in sth_iterate: the multi-step
       // kernels assume data this library wrote (Life: bytes already 0 or 1)
       if (int rc = sth::run_plan(q.plan[q.cur], st)) return rc;
       q.cur ^= 1;
@@ -302,17 +302,21 @@ struct sth_server {
       n -= 1;
     }
     const int64_t rem = q.r.steps - q.done;
-    const int64_t G = std::max<int32_t>(1, q.plan[0].fused_gens);  // steps per fused launch
-    const int64_t fused = n == rem ? std::max<int64_t>(0, (n - 2) / G) : n / G;
-    for (int64_t i = 0; i < fused; ++i) {
-      if (int rc = sth::run_fused(q.plan[q.cur], st)) return rc;
+    const int64_t G = std::max<int32_t>(1, q.plan[0].fused_gens);  // (most) steps per fused launch
+    const bool any = q.plan[0].fused_any && q.plan[1].fused_any;
+    int64_t left = n == rem ? std::max<int64_t>(0, n - 2) : n;
+    while (left >= (any ? 2 : G)) {
+      const int64_t k = (left + G - 1) / G, g = any ? (left + k - 1) / k : G;  // k launches of about equal length
+      if (int rc = sth::run_fused(q.plan[q.cur], st, g)) return rc;
       q.cur ^= 1;
-      q.done += G;
+      q.done += g;
+      left -= g;
+      n -= g;
       *launches += 1;
       solo_launches += 1;
       fused_launches += 1;
     }
-    for (int64_t i = G * fused; i < n; ++i) {
+    for (int64_t i = 0; i < n; ++i) {
       if (int rc = sth::run_plan(q.plan[q.cur], st)) return rc;
       q.cur ^= 1;
       q.done += 1;
