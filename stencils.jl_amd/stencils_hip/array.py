@@ -61,14 +61,24 @@ def colmajor_empty(shape, dtype, device, pitch=None, lead=0):
 
     `pitch` (elements) pads the contiguous dim of the allocation; `lead`
     elements precede the first element (used to align Halo interiors)."""
-    torch = _torch()
+    return _colmajor(shape, dtype, device, _torch().zeros, pitch, lead)
+
+
+def colmajor_uninit(shape, dtype, device):
+    """colmajor_empty without the zero fill, for a result that a kernel writes
+    whole: the fill is a launch of its own and one more pass over the result
+    (Mean over Window(1), f64 8191 x 8005: 114 of 308 us)."""
+    return _colmajor(shape, dtype, device, _torch().empty)
+
+
+def _colmajor(shape, dtype, device, alloc, pitch=None, lead=0):
     shape = tuple(int(s) for s in shape)
     p0 = shape[0] if pitch is None else int(pitch)
     rest = 1
     for s in shape[1:]:
         rest *= s
     total = lead + p0 * rest
-    buf = torch.zeros(max(total, 1), dtype=dtype, device=device)
+    buf = alloc(max(total, 1), dtype=dtype, device=device)
     strides = [1]
     acc = p0
     for s in shape[1:]:

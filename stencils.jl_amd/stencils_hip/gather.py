@@ -21,7 +21,7 @@ import numpy as np
 
 from . import _abi, _lib
 from .array import (AbstractStencilArray, StencilArray, SwitchingStencilArray,
-                    colmajor_copy, colmajor_empty, is_device, sth_dtype_of,
+                    colmajor_copy, colmajor_empty, colmajor_uninit, is_device, sth_dtype_of,
                     torch_dtype, to_numpy)
 from .boundary import Conditional, Halo, Remove, Use
 from .ops import Center, Reduction, Scaled, Terms, Unsupported, integer_fold_wraps, resolve
@@ -386,8 +386,9 @@ def gatherstencil_(f, dest, source=None, *args, flags: int = 0):
 
 
 def _alloc_like(parent, dt_code: int, shape):
+    """The result of a gather, which writes every cell of it."""
     if is_device(parent):
-        return colmajor_empty(shape, torch_dtype(dt_code), parent.device)
+        return colmajor_uninit(shape, torch_dtype(dt_code), parent.device)
     return np.zeros(shape, dtype=_abi.STH_TO_NUMPY[dt_code], order="F")
 
 
