@@ -264,7 +264,7 @@ def gen_runtime_tu(ctype: str) -> str:
 JIT_HEADERS = [("stencils_hip.h", REPO / "include" / "stencils_hip.h"), ("common.hpp", CSRC / "common.hpp"),
                ("tile_kernel.hpp", CSRC / "tile_kernel.hpp"), ("stream_kernel.hpp", CSRC / "stream_kernel.hpp"),
                ("zmarch2_kernel.hpp", CSRC / "zmarch2_kernel.hpp"), ("ymarch_kernel.hpp", CSRC / "ymarch_kernel.hpp"),
-               ("scatter_kernel.hpp", CSRC / "scatter_kernel.hpp")]
+               ("scatter_kernel.hpp", CSRC / "scatter_kernel.hpp"), ("bytes_kernel.hpp", CSRC / "bytes_kernel.hpp")]
 JIT_OPTIONS = [f for f in CXXFLAGS if f not in ("-fPIC", "-Wno-unused-command-line-argument") and not f.startswith("-I")]
 
 

@@ -319,6 +319,21 @@ inline const JitKernel* jit_stream_kernel(int dtype, int opk, int L, const int8_
                   "stream" + std::to_string(v) + "x" + std::to_string(ky), why);
 }
 
+// The one-byte extremes kernel (bytes_kernel) specialised to one shape.
+inline const JitKernel* jit_bytes_kernel(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int ky,
+                                         std::string* why) {
+  const char* tn = jit_type_name(dtype);
+  if (!tn) {
+    *why = "no type name";
+    return nullptr;
+  }
+  const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " + std::to_string(ky);
+  const std::string src = "#include \"bytes_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, 0) +
+                          "namespace sth {\ntemplate __global__ void bytes_kernel<" + targs +
+                          ">(MapParams);\n}  // namespace sth\n";
+  return jit_load(src, "&sth::bytes_kernel<" + targs + ">", "bytes" + std::to_string(ky), why);
+}
+
 // One pass of a multi-array gather as a streaming kernel over one stencil
 // argument: its fold f (scaled by its coefficient when `scaled`), combined
 // into the running value -- read back from dest (`acc_in`), or started from
