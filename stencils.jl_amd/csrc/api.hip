@@ -13,6 +13,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "batch_kernel.hpp"
@@ -250,6 +251,25 @@ int64_t zm2_extent(const DevArr& a, int64_t esize) {
   return ((a.n2 - 1) * a.s2 + (a.n1 - 1) * a.s1 + a.n0) * esize;
 }
 
+// Entries of one of the kernel catalogues (filled at load time, hundreds of
+// entries long) by element type, op and stencil length, in the catalogue's
+// order: a call looks at the few that can match.
+template <class E>
+const std::vector<const E*>& catalogue(const std::vector<E>& all, int dtype, int op, int L) {
+  using Index = std::unordered_map<uint64_t, std::vector<const E*>>;
+  auto key = [](int t, int o, int l) {
+    return static_cast<uint64_t>(t) << 48 | static_cast<uint64_t>(o) << 32 | static_cast<uint32_t>(l);
+  };
+  static const Index index = [&] {
+    Index m;
+    for (const E& e : all) m[key(e.dtype, e.op, e.L)].push_back(&e);
+    return m;
+  }();
+  static const std::vector<const E*> none;
+  const auto it = index.find(key(dtype, op, L));
+  return it == index.end() ? none : it->second;
+}
+
 int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st, int32_t bc,
               const void* padval, int32_t padding, const sth_op* op, uint32_t flags, Plan* out,
               std::vector<Variant>* cands_out = nullptr, std::string* group_out = nullptr) {
@@ -472,8 +492,9 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
   } else {
     if (!(flags & STH_GENERIC)) {
       std::string family;  // shapes with equal offsets (e.g. Window(1), Circle(1)) share kernels
-      for (const auto& e : registry()) {
-        if (e.L == 0 || e.dtype != sdt || e.op != op->kind || e.L != L || e.ndim != st->ndim) continue;
+      for (const KernelEntry* ep : catalogue(registry(), sdt, op->kind, L)) {
+        const KernelEntry& e = *ep;
+        if (e.ndim != st->ndim) continue;
         if (!offsets_equal(e.offs, L, offs3)) continue;
         const char* slash = std::strchr(e.name, '/');
         const std::string fam(e.name, slash ? static_cast<size_t>(slash - e.name) : std::strlen(e.name));
@@ -531,9 +552,9 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       if (L > kMaxRuntimeL) return fail(STH_ENOTSUP, "stencil with %d offsets (runtime max %d)", L, kMaxRuntimeL);
       const int cfg = reach[2] > 0 ? CFG_RT3D : (n[1] == 1 && reach[1] == 0 ? CFG_RT1D : CFG_RT2D);
       const KernelEntry* pick = nullptr;
-      for (const auto& e : registry())
-        if (e.L == 0 && e.dtype == sdt && e.op == op->kind && e.cfg == cfg) {
-          pick = &e;
+      for (const KernelEntry* e : catalogue(registry(), sdt, op->kind, 0))
+        if (e->cfg == cfg) {
+          pick = e;
           break;
         }
       if (!pick) return fail(STH_ENOTSUP, "no kernel for dtype %d op %d", sdt, op->kind);
@@ -622,8 +643,9 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= 3 && n[1] >= 3 && n[2] >= 3 &&
       n[0] * n[1] * n[2] >= fuse3d_min &&
       zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes && zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes) {
-    for (const auto& e : fused2_registry()) {
-      if (e.dtype != sdt || e.op != op->kind || e.L != L || e.ndim != st->ndim) continue;
+    for (const Fused2Entry* ep : catalogue(fused2_registry(), sdt, op->kind, L)) {
+      const Fused2Entry& e = *ep;
+      if (e.ndim != st->ndim) continue;
       if (!offsets_equal(e.offs, L, offs3)) continue;
       static const int64_t zm_waves = [] {
         const char* v = std::getenv("STH_ZM2_WAVES");
@@ -671,8 +693,9 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       n[0] * n[1] >= fuse2d_min &&
       sdt == odt && rows4(pl.p.src, dtype_size(sdt)) && rows4(pl.p.dst, dtype_size(odt)) &&
       zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes && zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes) {
-    for (const auto& e : fused2_registry()) {
-      if (e.dtype != sdt || e.op != op->kind || e.L != L || e.ndim != 2) continue;
+    for (const Fused2Entry* ep : catalogue(fused2_registry(), sdt, op->kind, L)) {
+      const Fused2Entry& e = *ep;
+      if (e.ndim != 2) continue;
       if (!offsets_equal(e.offs, L, offs3)) continue;
       pl.fn_fused = e.fn;
       pl.fused_gens = e.rows;
@@ -701,8 +724,9 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
   // the batched kernel's variant for this (dtype, op, offsets), if any
   pl.dtype = sdt;
   pl.bvariant = -1;
-  for (const auto& bv : batch_variants()) {
-    if (bv.dtype != sdt || bv.op != op->kind || bv.L != L || bv.ndim != st->ndim) continue;
+  for (const BatchVariant* bp : catalogue(batch_variants(), sdt, op->kind, L)) {
+    const BatchVariant& bv = *bp;
+    if (bv.ndim != st->ndim) continue;
     if (!offsets_equal(bv.offs, L, offs3)) continue;
     pl.bvariant = bv.variant;
     pl.bsv = bv.sv;
@@ -1115,8 +1139,10 @@ int with_device_table(sth_ctx* ctx, const void* data, size_t bytes, hipStream_t 
 // One step of many independent calls: calls with a batched variant go into
 // one launch per (element type, shape, reduction) after their halo refresh;
 // the rest, and calls that fill the device alone, run as single launches.
-// The job tables are uploaded into device slots the context owns.  With
-// more than one launch, the launches are spread over the context's batch
+// The job tables go up as one, into a device slot the context owns, before
+// the fork, so the launches need no upload, wait or event of their own (60
+// arrays in 9 groups: 202 us a call, bound by the host, with a table per
+// group).  With more than one launch, the launches are spread over the context's batch
 // streams (largest first, each to the least loaded stream) between a fork
 // and a join on `s`, so one launch's tail overlaps the next launch's start.
 int launch_batched(sth_ctx* ctx, const Plan* const* plans, int32_t n, bool serial_only, hipStream_t s) {
@@ -1126,60 +1152,71 @@ int launch_batched(sth_ctx* ctx, const Plan* const* plans, int32_t n, bool seria
   // the unbatched path keeps one launch per call, in order, on `s`
   int rc = group_batched(ctx, plans, n, serial_only, s, &groups, serial_only ? nullptr : &alone, &gcost);
   if (rc) return rc;
-  auto launch_group = [&](BatchGroups::value_type& kv, hipStream_t st) -> int {
-    std::vector<BatchJob>& bj = kv.second;
-    const BatchKernelEntry* ke = nullptr;
-    BatchParams bp;
-    int64_t blocks = 0;
-    int r2 = prepare_group(kv.first, bj, &ke, &bp, &blocks);
-    if (r2) return r2;
-    if (bp.total_tiles == 0) return STH_OK;
-    return with_device_table(ctx, bj.data(), bj.size() * sizeof(BatchJob), st, [&](const void* dev) {
-      bp.jobs = static_cast<const BatchJob*>(dev);
-      ke->fn(bp, static_cast<unsigned>(blocks), st);
-    });
-  };
-  // the launches, most costly first
+  // the launches, most costly first; the groups' job tables one after another
   struct Item {
     const Plan* alone;
-    BatchGroups::value_type* group;
+    const BatchKernelEntry* ke;
+    BatchParams bp;
+    int64_t blocks;
+    size_t first;  // of its jobs in the table
     double cost;
   };
   std::vector<Item> items;
-  for (const Plan* pl : alone) items.push_back({pl, nullptr, plan_cost(*pl)});
-  for (auto& kv : groups) items.push_back({nullptr, &kv, gcost[kv.first]});
+  std::vector<BatchJob> table;
+  for (const Plan* pl : alone) items.push_back({pl, nullptr, BatchParams{}, 0, 0, plan_cost(*pl)});
+  for (auto& kv : groups) {
+    Item it{nullptr, nullptr, BatchParams{}, 0, table.size(), gcost[kv.first]};
+    if ((rc = prepare_group(kv.first, kv.second, &it.ke, &it.bp, &it.blocks))) return rc;
+    if (it.bp.total_tiles == 0) continue;
+    table.insert(table.end(), kv.second.begin(), kv.second.end());
+    items.push_back(it);
+  }
+  if (items.empty()) return STH_OK;
   std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.cost > b.cost; });
-  auto run_item = [&](const Item& it, hipStream_t st) -> int {
-    return it.alone ? run_plan(*it.alone, st) : launch_group(*it.group, st);
-  };
-  const int nst = batch_streams_wanted();
-  if (items.size() <= 1 || nst <= 1) {
-    for (const Item& it : items)
-      if ((rc = run_item(it, s))) return rc;
-    return STH_OK;
-  }
-  std::lock_guard<std::mutex> fork_lock(ctx->batch_mu);
-  if ((rc = ensure_batch_streams(ctx, nst))) return rc;
-  STH_HIP(hipEventRecord(ctx->batch_fork, s));
-  double load[kBatchStreams] = {};
-  bool used[kBatchStreams] = {};
-  for (const Item& it : items) {
-    int k = 0;
-    for (int i = 1; i < nst; ++i)
-      if (load[i] < load[k]) k = i;
-    if (!used[k]) {
-      STH_HIP(hipStreamWaitEvent(ctx->batch_streams[k], ctx->batch_fork, 0));
-      used[k] = true;
+  auto run_all = [&](const void* dev) -> int {
+    auto run_item = [&](const Item& it, hipStream_t st) -> int {
+      if (it.alone) return run_plan(*it.alone, st);
+      BatchParams bp = it.bp;
+      bp.jobs = static_cast<const BatchJob*>(dev) + it.first;
+      it.ke->fn(bp, static_cast<unsigned>(it.blocks), st);
+      STH_HIP(hipGetLastError());
+      return STH_OK;
+    };
+    const int nst = batch_streams_wanted();
+    if (items.size() <= 1 || nst <= 1) {
+      for (const Item& it : items)
+        if (int r2 = run_item(it, s)) return r2;
+      return STH_OK;
     }
-    load[k] += it.cost;
-    if ((rc = run_item(it, ctx->batch_streams[k]))) return rc;
-  }
-  for (int k = 0; k < nst; ++k) {
-    if (!used[k]) continue;
-    STH_HIP(hipEventRecord(ctx->batch_join[k], ctx->batch_streams[k]));
-    STH_HIP(hipStreamWaitEvent(s, ctx->batch_join[k], 0));
-  }
-  return STH_OK;
+    if (int r2 = ensure_batch_streams(ctx, nst)) return r2;
+    STH_HIP(hipEventRecord(ctx->batch_fork, s));
+    double load[kBatchStreams] = {};
+    bool used[kBatchStreams] = {};
+    int err = STH_OK;
+    for (const Item& it : items) {
+      int k = 0;
+      for (int i = 1; i < nst; ++i)
+        if (load[i] < load[k]) k = i;
+      if (!used[k]) {
+        STH_HIP(hipStreamWaitEvent(ctx->batch_streams[k], ctx->batch_fork, 0));
+        used[k] = true;
+      }
+      load[k] += it.cost;
+      if ((err = run_item(it, ctx->batch_streams[k]))) break;  // the join still covers what was launched
+    }
+    for (int k = 0; k < nst; ++k) {
+      if (!used[k]) continue;
+      STH_HIP(hipEventRecord(ctx->batch_join[k], ctx->batch_streams[k]));
+      STH_HIP(hipStreamWaitEvent(s, ctx->batch_join[k], 0));
+    }
+    return err;
+  };
+  std::lock_guard<std::mutex> fork_lock(ctx->batch_mu);
+  if (table.empty()) return run_all(nullptr);
+  int err = STH_OK;
+  rc = with_device_table(ctx, table.data(), table.size() * sizeof(BatchJob), s,
+                         [&](const void* dev) { err = run_all(dev); });
+  return err ? err : rc;
 }
 
 // The same step with every job table in `table` (the device's fixed

@@ -300,38 +300,84 @@ inline const JitKernel* jit_load(const std::string& src, const std::string& expr
   return &jk;
 }
 
+// A specialisation already loaded, by what it was asked for: the kernel's
+// kind and its parameters as bytes, so that a call need not write out the
+// source to look it up.  A kernel that could not be built or loaded is not
+// kept here.
+struct JitRequest {
+  std::string key;
+  explicit JitRequest(char kind) {
+    int dev = -1;
+    (void)hipGetDevice(&dev);
+    key.push_back(kind);
+    add(dev);
+  }
+  JitRequest& add(int v) {
+    key.append(reinterpret_cast<const char*>(&v), sizeof v);
+    return *this;
+  }
+  template <class T>
+  JitRequest& add(const T* v, size_t n) {
+    add(static_cast<int>(n));
+    key.append(reinterpret_cast<const char*>(v), n * sizeof(T));
+    return *this;
+  }
+};
+template <class Build>
+inline const JitKernel* jit_remembered(const JitRequest& r, Build&& build) {
+  static std::mutex m;
+  static std::map<std::string, const JitKernel*> known;
+  {
+    std::lock_guard<std::mutex> lk(m);
+    const auto it = known.find(r.key);
+    if (it != known.end()) return it->second;
+  }
+  const JitKernel* k = build();
+  if (k) {
+    std::lock_guard<std::mutex> lk(m);
+    known.emplace(r.key, k);
+  }
+  return k;
+}
+
 // The streaming kernel specialised to one shape (L offsets, x fastest, as
 // int8 triples) for storage type `dtype`, fold `opk`, V cells per lane and
 // KY rows per lane, loaded on the current device.
 inline const JitKernel* jit_stream_kernel(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz,
                                           int v, int ky, std::string* why) {
-  const char* tn = jit_type_name(dtype);
-  if (!tn) {
-    *why = "no type name";
-    return nullptr;
-  }
-  const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " +
-                            std::to_string(v) + ", " + std::to_string(ky);
-  const std::string src = "#include \"stream_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, rz) +
-                          "namespace sth {\ntemplate __global__ void stream_kernel<" + targs +
-                          ">(MapParams);\n}  // namespace sth\n";
-  return jit_load(src, "&sth::stream_kernel<" + targs + ">",
-                  "stream" + std::to_string(v) + "x" + std::to_string(ky), why);
+  const JitRequest request = JitRequest('s').add(dtype).add(opk).add(rx).add(ry).add(rz).add(v).add(ky).add(offs3, 3 * static_cast<size_t>(L));
+  return jit_remembered(request, [&]() -> const JitKernel* {
+    const char* tn = jit_type_name(dtype);
+    if (!tn) {
+      *why = "no type name";
+      return nullptr;
+    }
+    const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " +
+                              std::to_string(v) + ", " + std::to_string(ky);
+    const std::string src = "#include \"stream_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, rz) +
+                            "namespace sth {\ntemplate __global__ void stream_kernel<" + targs +
+                            ">(MapParams);\n}  // namespace sth\n";
+    return jit_load(src, "&sth::stream_kernel<" + targs + ">",
+                    "stream" + std::to_string(v) + "x" + std::to_string(ky), why);
+  });
 }
 
 // The one-byte extremes kernel (bytes_kernel) specialised to one shape.
 inline const JitKernel* jit_bytes_kernel(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int ky,
                                          std::string* why) {
-  const char* tn = jit_type_name(dtype);
-  if (!tn) {
-    *why = "no type name";
-    return nullptr;
-  }
-  const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " + std::to_string(ky);
-  const std::string src = "#include \"bytes_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, 0) +
-                          "namespace sth {\ntemplate __global__ void bytes_kernel<" + targs +
-                          ">(MapParams);\n}  // namespace sth\n";
-  return jit_load(src, "&sth::bytes_kernel<" + targs + ">", "bytes" + std::to_string(ky), why);
+  const JitRequest request = JitRequest('b').add(dtype).add(opk).add(rx).add(ry).add(ky).add(offs3, 3 * static_cast<size_t>(L));
+  return jit_remembered(request, [&]() -> const JitKernel* {
+    const char* tn = jit_type_name(dtype);
+    if (!tn) {
+      *why = "no type name";
+      return nullptr;
+    }
+    const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " + std::to_string(ky);
+    const std::string src = "#include \"bytes_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, 0) +
+                            "namespace sth {\ntemplate __global__ void bytes_kernel<" + targs +
+                            ">(MapParams);\n}  // namespace sth\n";
+    return jit_load(src, "&sth::bytes_kernel<" + targs + ">", "bytes" + std::to_string(ky), why);
+  });
 }
 
 // One pass of a multi-array gather as a streaming kernel over one stencil
@@ -453,13 +499,19 @@ inline bool jit_multi_source(int dtype, int opk, int L, const int8_t* offs3, int
 
 inline const JitKernel* jit_multi_pass(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz, int v,
                                        int ky, bool acc_in, const std::string& items, bool mul, std::string* why) {
-  static_assert(sizeof(MultiEpiParams) == 8 + 16 + 64 + 128 + 64, "epilogue parameter layout");
-  std::string src, expr;
-  if (!jit_multi_source(dtype, opk, L, offs3, rx, ry, rz, v, ky, acc_in, items, mul, &src, &expr)) {
-    *why = "no type name";
-    return nullptr;
-  }
-  return jit_load(src, expr, "multi" + std::to_string(v) + "x" + std::to_string(ky), why);
+  const JitRequest request = JitRequest('m')
+                                 .add(dtype).add(opk).add(rx).add(ry).add(rz).add(v).add(ky).add(acc_in).add(mul)
+                                 .add(items.data(), items.size())
+                                 .add(offs3, 3 * static_cast<size_t>(L));
+  return jit_remembered(request, [&]() -> const JitKernel* {
+    static_assert(sizeof(MultiEpiParams) == 8 + 16 + 64 + 128 + 64, "epilogue parameter layout");
+    std::string src, expr;
+    if (!jit_multi_source(dtype, opk, L, offs3, rx, ry, rz, v, ky, acc_in, items, mul, &src, &expr)) {
+      *why = "no type name";
+      return nullptr;
+    }
+    return jit_load(src, expr, "multi" + std::to_string(v) + "x" + std::to_string(ky), why);
+  });
 }
 
 // A stencil argument of a fused multi-array kernel: its fold and shape.
@@ -608,12 +660,15 @@ inline bool jit_fused_source(int dtype, int opk, int L, const int8_t* offs3, int
 
 inline const JitKernel* jit_fused_kernel(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz,
                                          int ndim, int bc, std::string* why) {
-  std::string src, expr;
-  if (!jit_fused_source(dtype, opk, L, offs3, rx, ry, rz, ndim, bc, &src, &expr)) {
-    *why = "no type name";
-    return nullptr;
-  }
-  return jit_load(src, expr, ndim == 3 ? "zmarch2" : "ymarch", why);
+  const JitRequest request = JitRequest('f').add(dtype).add(opk).add(rx).add(ry).add(rz).add(ndim).add(bc).add(offs3, 3 * static_cast<size_t>(L));
+  return jit_remembered(request, [&]() -> const JitKernel* {
+    std::string src, expr;
+    if (!jit_fused_source(dtype, opk, L, offs3, rx, ry, rz, ndim, bc, &src, &expr)) {
+      *why = "no type name";
+      return nullptr;
+    }
+    return jit_load(src, expr, ndim == 3 ? "zmarch2" : "ymarch", why);
+  });
 }
 
 // The scatter kernel with the interior order of each dest-column residue as
@@ -653,12 +708,15 @@ inline bool jit_scatter_source(int dtype, int kind, int combine, int S, int L, c
 
 inline const JitKernel* jit_scatter_kernel(int dtype, int kind, int combine, int S, int L, const int32_t* deltas,
                                            std::string* why) {
-  std::string src, expr;
-  if (!jit_scatter_source(dtype, kind, combine, S, L, deltas, &src, &expr)) {
-    *why = "no specialisation for this element type";
-    return nullptr;
-  }
-  return jit_load(src, expr, "scatter", why);
+  const JitRequest request = JitRequest('c').add(dtype).add(kind).add(combine).add(S).add(deltas, static_cast<size_t>(S) * L);
+  return jit_remembered(request, [&]() -> const JitKernel* {
+    std::string src, expr;
+    if (!jit_scatter_source(dtype, kind, combine, S, L, deltas, &src, &expr)) {
+      *why = "no specialisation for this element type";
+      return nullptr;
+    }
+    return jit_load(src, expr, "scatter", why);
+  });
 }
 
 // Launch a loaded specialisation with the call's parameters (one block of

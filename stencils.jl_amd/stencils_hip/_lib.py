@@ -108,7 +108,7 @@ def load_library(path: Path | None = None):
 
 
 def lib():
-    return load_library()
+    return _lib if _lib is not None else load_library()
 
 
 def check(status: int):

@@ -22,12 +22,17 @@ def _torch():
     return torch
 
 
+_TENSOR = None
+
+
 def is_device(x) -> bool:
-    try:
-        torch = _torch()
-    except ImportError:  # pragma: no cover
-        return False
-    return isinstance(x, torch.Tensor)
+    global _TENSOR
+    if _TENSOR is None:
+        try:
+            _TENSOR = _torch().Tensor
+        except ImportError:  # pragma: no cover
+            return False
+    return type(x) is _TENSOR or isinstance(x, _TENSOR)
 
 
 TORCH_DTYPES = None
@@ -35,9 +40,9 @@ TORCH_DTYPES = None
 
 def sth_dtype_of(x) -> int:
     if is_device(x):
-        torch = _torch()
         global TORCH_DTYPES
         if TORCH_DTYPES is None:
+            torch = _torch()
             TORCH_DTYPES = {
                 torch.bool: _abi.BOOL, torch.uint8: _abi.U8, torch.int8: _abi.I8,
                 torch.uint16: _abi.U16, torch.int16: _abi.I16, torch.uint32: _abi.U32,
@@ -49,11 +54,14 @@ def sth_dtype_of(x) -> int:
     return _abi.NUMPY_TO_STH[np.dtype(x.dtype)]
 
 
+_STH_TO_TORCH: dict = {}
+
+
 def torch_dtype(code: int):
-    torch = _torch()
-    sth_dtype_of(torch.empty(0))  # fill the table
-    inv = {v: k for k, v in TORCH_DTYPES.items()}
-    return inv[code]
+    if not _STH_TO_TORCH:
+        sth_dtype_of(_torch().empty(0))  # fill the table
+        _STH_TO_TORCH.update({v: k for k, v in TORCH_DTYPES.items()})
+    return _STH_TO_TORCH[code]
 
 
 def colmajor_empty(shape, dtype, device, pitch=None, lead=0):
@@ -68,7 +76,13 @@ def colmajor_uninit(shape, dtype, device):
     """colmajor_empty without the zero fill, for a result that a kernel writes
     whole: the fill is a launch of its own and one more pass over the result
     (Mean over Window(1), f64 8191 x 8005: 114 of 308 us)."""
-    return _colmajor(shape, dtype, device, _torch().empty)
+    strides, total = [], 1
+    for s in shape:
+        strides.append(total)
+        total *= int(s)
+    if total == 0:  # an empty result still has an address
+        return _colmajor(shape, dtype, device, _torch().empty)
+    return _torch().empty_strided(tuple(shape), strides, dtype=dtype, device=device)
 
 
 def _colmajor(shape, dtype, device, alloc, pitch=None, lead=0):
@@ -106,12 +120,12 @@ def to_numpy(t):
 
 def elem_strides(x):
     if is_device(x):
-        return tuple(int(s) for s in x.stride())
+        return x.stride()
     return tuple(s // x.itemsize for s in x.strides)
 
 
 def data_ptr(x) -> int:
-    return int(x.data_ptr()) if is_device(x) else int(x.ctypes.data)
+    return x.data_ptr() if is_device(x) else int(x.ctypes.data)
 
 
 def halo_pitch(n0: int, R: int, esize: int, align: int = 64):

@@ -16,6 +16,7 @@ There is no CPU path: without the HIP library or a device the call raises.
 from __future__ import annotations
 
 import ctypes
+import struct
 
 import numpy as np
 
@@ -46,6 +47,27 @@ class _Call:
         return x
 
 
+def _padval_plain(pv, dt: int):
+    """The bytes of a plain Python number that an element of type `dt` holds
+    exactly, or None (numpy decides: 4 us, this 0.5)."""
+    try:
+        if type(pv) is float:
+            if dt == _abi.F64:
+                return struct.pack("=d", pv) if pv == pv else None
+            if dt == _abi.F32:
+                b = struct.pack("=f", pv)
+                return b if struct.unpack("=f", b)[0] == pv else None
+        elif type(pv) is int and dt in _INT_FORMATS:
+            return struct.pack(_INT_FORMATS[dt], pv)
+    except (OverflowError, struct.error):
+        pass
+    return None
+
+
+_INT_FORMATS = {_abi.U8: "=B", _abi.I8: "=b", _abi.U16: "=H", _abi.I16: "=h", _abi.U32: "=I", _abi.I32: "=i",
+                _abi.U64: "=Q", _abi.I64: "=q"}
+
+
 def _padval_bytes(sa: AbstractStencilArray):
     bc = sa.boundary
     if not isinstance(bc, Remove):
@@ -63,6 +85,9 @@ def _padval_bytes(sa: AbstractStencilArray):
         if float(t[0]) != float(pv):
             raise Unsupported("padval is not representable in the storage type")
         return t.view(torch.int16).numpy().tobytes()
+    b = _padval_plain(pv, dt)
+    if b is not None:
+        return b
     npdt = _abi.STH_TO_NUMPY[dt]
     v = np.array(pv).astype(npdt)
     if not (v == np.array(pv)).all() or (dt not in _abi.FLOAT_DTYPES and isinstance(pv, float)):
@@ -150,16 +175,12 @@ def _device_index(x) -> int:
 
 
 def _stream(dev: int):
-    return ctypes.c_void_p(_torch().cuda.current_stream(dev).cuda_stream)
-
-
-def _raw_stream(dev: int):
     """The current stream of `dev` as a hipStream_t (torch's raw getter when
     it has one: no Stream object per call)."""
     torch = _torch()
     get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
     if get is None:
-        return _stream(dev)
+        return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
     return ctypes.c_void_p(get(dev))
 
 
@@ -492,7 +513,7 @@ def mapstencil_steps(f, A: SwitchingStencilArray, steps: int, graph: bool = True
     fl = flags | (_abi.GRAPH if graph else 0)
     _lib.check(_lib.lib().sth_iterate(ctx, ctypes.byref(da), ctypes.byref(db), ctypes.byref(st),
                                       A.boundary.code, pvbuf, A.padding.code, ctypes.byref(op),
-                                      int(steps), fl, ctypes.byref(cur), _raw_stream(dev)))
+                                      int(steps), fl, ctypes.byref(cur), _stream(dev)))
     if host:
         A.source[...] = to_numpy(a)
         A.dest[...] = to_numpy(b)
@@ -614,7 +635,7 @@ def mapstencil_steps_batch(items, graph: bool = True, serial: bool = False, flag
     if n == 0:
         return []
     fl = flags | (_abi.GRAPH if graph else 0) | (_abi.BATCH_SERIAL if serial else 0)
-    _lib.check(_lib.lib().sth_iterate_batch(_lib.context(dev), n, jobs, steps, fl, cur, _raw_stream(dev)))
+    _lib.check(_lib.lib().sth_iterate_batch(_lib.context(dev), n, jobs, steps, fl, cur, _stream(dev)))
     return [A.switch() if cur[i] == 1 else A for i, (_, A, _k) in enumerate(items)]
 
 
