@@ -198,8 +198,8 @@ def shape_struct(st) -> tuple[str, int, tuple[int, int, int]]:
 
 # Every (shape, op) of the catalogue gets its own batched kernel: one op's
 # streaming body per kernel keeps the code small (instruction cache) and the
-# register count that of that body; a batch launches once per (element type,
-# shape, op) present.  Batch translation units are grouped per shape.
+# register count that of that body; a batch of one 2-D variant, and 3-D ones,
+# launch it.  Batch translation units are grouped per shape.
 BATCH_SHAPES = [shape_name(st) for st, _ in CATALOG]
 
 
@@ -232,8 +232,39 @@ def gen_batch_tu(ctype: str, code: str, shape: str) -> str:
             regs.append(f"  batch_variants().push_back(BatchVariant{{{code}, {op}, {L}, {st.N}, "
                         f"&Shape_{shape}::off[0][0], {v}, {sv}, {sky}, {v}}});")
             regs.append(f"  batch_kernels().push_back(BatchKernelEntry{{{code}, {v}, "
-                        f"&launch_batch<{ctype}, {disp}>, &batch_occupancy<{ctype}, {disp}>}});")
+                        f"&launch_batch<{ctype}, {disp}>, {st.N}}});")
     lines += ["struct Init {", "  Init() {", *regs, "  }", "} init;",
+              "}  // namespace", "}  // namespace sth", ""]
+    return "\n".join(lines)
+
+
+def gen_batch_all_tu(ctype: str, code: str) -> str:
+    """One kernel that runs any 2-D variant of the catalogue, chosen per job:
+    a batch of several variants is one launch."""
+    lines = [
+        f"// Generated by stencils.jl_amd/build.py: the batched kernel of every 2-D variant for {ctype}.",
+        '#include "batch_kernel.hpp"',
+        "namespace sth {",
+        "namespace {",
+    ]
+    cases = []
+    for idx, (st, ops) in enumerate(CATALOG):
+        if st.N != 2:
+            continue
+        text, _, _ = shape_struct(st)
+        lines.append(text)
+        sv, sky = stream_variants(ctype, st)[0]
+        for k, op in enumerate(batch_ops(ops)):
+            cases.append(f"      case {100 * (idx + 1) + k}: stream_body<{ctype}, {op}, Shape_{shape_name(st)}, {sv}, "
+                         f"{sky}>(j, bx, by, bz, lane, wave); break;")
+    lines += [f"struct Dispatch_{ctype}_all {{",
+              "  __device__ static __forceinline__ void run(const BatchJob& j, int bx, int by, int bz, int lane, "
+              "int wave) {",
+              "    switch (j.variant) {", *cases, "      default: break;", "    }", "  }", "};",
+              "struct Init {", "  Init() {",
+              f"    batch_kernels().push_back(BatchKernelEntry{{{code}, kBatchAll, "
+              f"&launch_batch_all<{ctype}, Dispatch_{ctype}_all>, 2}});",
+              "  }", "} init;",
               "}  // namespace", "}  // namespace sth", ""]
     return "\n".join(lines)
 
@@ -310,6 +341,9 @@ def sources():
             p = GEN / f"batch_{ctype}_{shape}.hip"
             write_if_changed(p, gen_batch_tu(ctype, code, shape))
             srcs.append(p)
+        p = GEN / f"batch_{ctype}_all.hip"
+        write_if_changed(p, gen_batch_all_tu(ctype, code))
+        srcs.insert(0, p)  # the longest to compile
     p = GEN / "jit_sources.hip"
     write_if_changed(p, gen_jit_tu())
     srcs.append(p)

@@ -1048,6 +1048,49 @@ int group_batched(sth_ctx* ctx, const Plan* const* plans, int32_t n, bool serial
   return STH_OK;
 }
 
+// Whether a batch of several 2-D variants is one launch (STH_BATCH_MERGE=0:
+// one launch per variant).
+bool batch_merge_enabled() {
+  static const bool v = [] {
+    const char* e = std::getenv("STH_BATCH_MERGE");
+    return !(e && std::strcmp(e, "0") == 0);
+  }();
+  return v;
+}
+
+// The 2-D groups of each element type that has several become one, which the
+// kernel of every 2-D variant runs, longest stencils first.
+void merge_groups(BatchGroups* groups, std::map<int64_t, double>* cost) {
+  std::map<int64_t, std::vector<int64_t>> keys;  // element type -> its 2-D groups
+  for (const auto& e : batch_kernels()) {
+    const int64_t key = static_cast<int64_t>(e.dtype) * 65536 + e.klass;
+    if (e.klass != kBatchAll && e.ndim == 2 && groups->count(key)) keys[e.dtype].push_back(key);
+  }
+  for (auto& kv : keys) {
+    std::vector<int64_t>& ks = kv.second;
+    if (ks.size() < 2) continue;
+    auto per_cell = [&](int64_t k) {
+      double cells = 0;
+      for (const BatchJob& j : (*groups)[k]) cells += static_cast<double>(j.src.n0) * j.src.n1 * j.src.n2;
+      return cells > 0 ? (*cost)[k] / cells : 0.0;
+    };
+    std::map<int64_t, double> weight;
+    for (int64_t k : ks) weight[k] = per_cell(k);
+    std::stable_sort(ks.begin(), ks.end(), [&](int64_t a, int64_t b) { return weight[a] > weight[b]; });
+    const int64_t all = kv.first * 65536 + kBatchAll;
+    std::vector<BatchJob> jobs;
+    double sum = 0;
+    for (int64_t k : ks) {
+      std::vector<BatchJob>& g = (*groups)[k];
+      jobs.insert(jobs.end(), g.begin(), g.end());
+      sum += (*cost)[k];
+      groups->erase(k);
+    }
+    (*groups)[all] = std::move(jobs);
+    (*cost)[all] = sum;
+  }
+}
+
 // Second half, per group: its kernel, the jobs' first tiles and the launch
 // shape (one tile per workgroup: a workgroup's tiles run one after another
 // with no overlap inside a wave; STH_BATCH_TPB sets strips).  Sets *total to
@@ -1136,15 +1179,17 @@ int with_device_table(sth_ctx* ctx, const void* data, size_t bytes, hipStream_t 
   return STH_OK;
 }
 
-// One step of many independent calls: calls with a batched variant go into
-// one launch per (element type, shape, reduction) after their halo refresh;
-// the rest, and calls that fill the device alone, run as single launches.
-// The job tables go up as one, into a device slot the context owns, before
-// the fork, so the launches need no upload, wait or event of their own (60
-// arrays in 9 groups: 202 us a call, bound by the host, with a table per
-// group).  With more than one launch, the launches are spread over the context's batch
-// streams (largest first, each to the least loaded stream) between a fork
-// and a join on `s`, so one launch's tail overlaps the next launch's start.
+// One step of many independent calls: after their halo refresh, the calls
+// with a 2-D batched variant go into one launch per element type, those with
+// a 3-D one into one per variant; the rest, and calls that fill the device
+// alone, run as single launches.  The job tables go up as one, into a device
+// slot the context owns, before the fork, so the launches need no upload,
+// wait or event of their own.  With more than one launch, the launches are
+// spread over the context's batch streams (largest first, each to the least
+// loaded stream) between a fork and a join on `s`, so one launch's tail
+// overlaps the next launch's start.  60 f32 arrays of 9 variants: 203 us a
+// call with a table and a launch per variant, 167 with one table (host 133
+// us), 95 with one launch (host 33 us).
 int launch_batched(sth_ctx* ctx, const Plan* const* plans, int32_t n, bool serial_only, hipStream_t s) {
   BatchGroups groups;
   std::vector<const Plan*> alone;
@@ -1164,6 +1209,7 @@ int launch_batched(sth_ctx* ctx, const Plan* const* plans, int32_t n, bool seria
   std::vector<Item> items;
   std::vector<BatchJob> table;
   for (const Plan* pl : alone) items.push_back({pl, nullptr, BatchParams{}, 0, 0, plan_cost(*pl)});
+  if (groups.size() > 1 && batch_merge_enabled()) merge_groups(&groups, &gcost);
   for (auto& kv : groups) {
     Item it{nullptr, nullptr, BatchParams{}, 0, table.size(), gcost[kv.first]};
     if ((rc = prepare_group(kv.first, kv.second, &it.ke, &it.bp, &it.blocks))) return rc;

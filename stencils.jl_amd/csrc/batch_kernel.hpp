@@ -1,5 +1,5 @@
 // Batched gather: many independent mapstencil calls of mixed sizes, shapes
-// and reductions in one launch per (element type, stencil shape, op).
+// and reductions in one launch.
 //
 // The host flattens the tiles of every job into one index space (job j owns
 // tiles [tile_begin_j, tile_begin_{j+1})) and launches one workgroup per
@@ -7,10 +7,12 @@
 // strips to CUs as they free up, so cheap and expensive jobs balance without
 // atomics or barriers (a single device-wide atomic tile counter measured much
 // slower: same-address atomics serialise in L2).  A workgroup finds its first
-// job by binary search over the job table (uniform, scalar loads) and walks
-// forward.  Each tile runs the streaming body of the kernel's (shape, op)
-// variant: one small kernel per variant keeps the code in the instruction
-// cache (a kernel switching over a shape's ops measured up to 40 % slower).
+// job in the job table and walks forward.  Each tile runs the streaming body
+// of the job's (shape, op) variant.  A batch of one variant, and 3-D ones,
+// run a kernel that holds this variant alone; 2-D jobs of several variants
+// run one kernel that holds them all and branches per tile (uniformly): a
+// launch per variant lasts as long as its slowest workgroup, with most of the
+// chip idle behind it, and costs the host a launch each.
 // Results are bit-identical to one sth_map call per job (same fold
 // expressions per cell).
 #pragma once
@@ -44,24 +46,32 @@ struct BatchParams {
 // kernel's variant; it is generated per (storage type, shape, op) and
 // force-inlined into the kernel, which makes no calls.
 template <typename S, class Dispatch>
-__global__ __launch_bounds__(256) void batch_kernel(BatchParams bp, const BatchJob* __restrict__ jobs) {
+__device__ __forceinline__ void batch_run(const BatchParams& bp, const BatchJob* __restrict__ jobs, int64_t b) {
   // `jobs` is read-only and aliases nothing the kernel writes, so its fields
   // stay in scalar registers instead of being reloaded after every store.
   const int lane = static_cast<int>(threadIdx.x) & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const int G = static_cast<int>(gridDim.x);
-  const int64_t b = xcd_block_id(static_cast<int>(blockIdx.x), G, 1);
   int64_t t = b * bp.tiles_per_block;
   const int64_t tend = t + bp.tiles_per_block < bp.total_tiles ? t + bp.tiles_per_block : bp.total_tiles;
   if (t >= tend) return;
-  // last job whose first tile is <= t
-  int lo = 0, hi = bp.njobs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (jobs[mid].tile_begin <= t) lo = mid;
-    else hi = mid - 1;
+  // The last job whose first tile is <= t: every lane looks at one job (at
+  // one range of jobs first, when they are many), one or two loads in a row
+  // where a binary search takes one per halving.
+  int j = 0;
+  if (bp.njobs > 64) {
+    const int step = (bp.njobs + 63) / 64;
+    const int i = lane * step;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(i < bp.njobs && jobs[i < bp.njobs ? i : 0].tile_begin <= t);
+    j = (63 - __builtin_clzll(m)) * step;  // job 0 starts at tile 0: m has a bit
   }
-  int j = lo;
+  for (bool more = true; more;) {
+    const int i = j + lane;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(i < bp.njobs && jobs[i < bp.njobs ? i : 0].tile_begin <= t);
+    const int last = 63 - __builtin_clzll(m);
+    j += last;
+    more = last == 63;  // (ends: the jobs do)
+  }
+  j = __builtin_amdgcn_readfirstlane(j);
   for (; t < tend; ++t) {
     while (j + 1 < bp.njobs && jobs[j + 1].tile_begin <= t) ++j;
     const BatchJob job = jobs[j];  // a register copy for the tile
@@ -74,6 +84,32 @@ __global__ __launch_bounds__(256) void batch_kernel(BatchParams bp, const BatchJ
     const int bz = static_cast<int>(byz / ty);
     Dispatch::run(job, bx, by, bz, lane, wave);
   }
+}
+
+template <typename S, class Dispatch>
+__global__ __launch_bounds__(256) void batch_kernel(BatchParams bp, const BatchJob* __restrict__ jobs) {
+  batch_run<S, Dispatch>(bp, jobs, xcd_block_id(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), 1));
+}
+
+// Every 2-D variant in one kernel.  Blocks go to the XCDs round robin: of
+// each 8 kBatchChunk consecutive strips an XCD takes kBatchChunk neighbours,
+// which share halo rows in its L2, and every XCD gets a share of each job
+// (one contiguous range per XCD would leave the long stencils to a few).
+// (60 f32 arrays of 64^2 .. 2048^2, 296 MB: 94 us with chunks of 16, 97 with
+// 4, 99 with 64; one launch per variant 150 us.)  Four waves per SIMD: 85 us
+// against 94 with the three that the longest stencils' registers leave;
+// 8-byte types would spill at four.
+constexpr int kBatchChunk = 16;
+template <typename S, class Dispatch>
+__global__ __launch_bounds__(256, sizeof(typename Elem<S>::raw) == 8 ? 3 : 4) void batch_all_kernel(BatchParams bp, const BatchJob* __restrict__ jobs) {
+  int64_t b = blockIdx.x;
+  constexpr int kSpan = 8 * kBatchChunk;
+  const int64_t span = b / kSpan * kSpan;
+  if (span + kSpan <= static_cast<int64_t>(gridDim.x)) {
+    const int r = static_cast<int>(b - span);
+    b = span + (r & 7) * kBatchChunk + (r >> 3);
+  }
+  batch_run<S, Dispatch>(bp, jobs, b);
 }
 
 using BatchLaunchFn = void (*)(const BatchParams&, unsigned blocks, hipStream_t);
@@ -89,11 +125,13 @@ struct BatchVariant {
   int klass;    // the batched kernel that runs this variant (one per variant)
 };
 
+constexpr int kBatchAll = 0;  // klass of the kernel that runs every 2-D variant (0 is no variant)
+
 struct BatchKernelEntry {
   int dtype;
   int klass;
   BatchLaunchFn fn;
-  int (*occupancy)();  // resident workgroups per CU
+  int ndim;  // stencil dims
 };
 
 std::vector<BatchVariant>& batch_variants();
@@ -105,11 +143,8 @@ void launch_batch(const BatchParams& bp, unsigned blocks, hipStream_t s) {
 }
 
 template <typename S, class Dispatch>
-int batch_occupancy() {
-  int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, batch_kernel<S, Dispatch>, 256, 0) != hipSuccess)
-    n = 1;
-  return n > 0 ? n : 1;
+void launch_batch_all(const BatchParams& bp, unsigned blocks, hipStream_t s) {
+  hipLaunchKernelGGL((batch_all_kernel<S, Dispatch>), dim3(blocks), dim3(256), 0, s, bp, bp.jobs);
 }
 
 }  // namespace sth
