@@ -124,6 +124,7 @@ def gen_static_tu(st, ops, ctype: str, code: str) -> str:
         '#include "zmarch2_kernel.hpp"',
         '#include "zmarch1_kernel.hpp"',
         '#include "ymarch_kernel.hpp"',
+        '#include "zmarch_kernel.hpp"',
         "namespace sth {",
         "namespace {",
         f"struct Shape_{name} {{",
@@ -157,6 +158,12 @@ def gen_static_tu(st, ops, ctype: str, code: str) -> str:
             f"&Shape_{name}::off[0][0], {fn}, \"{name}_{ctype}_{op}/lds\"}});")
         i += 1
         if st.N == 3 and max(rx, ry, rz) <= 1:
+            if all(sum(map(abs, o)) <= 1 for o in o3) and ESIZE[ctype] <= 4:
+                # up to four steps per launch (star stencils, 4-byte values)
+                lines.append(
+                    f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
+                    f"&Shape_{name}::off[0][0], &launch_zmarch<{ctype}, {op}, Shape_{name}>, kZmGens, 1}});")
+                i += 1
             # two steps per launch for iterations (3-D: march along z)
             lines.append(
                 f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
@@ -168,7 +175,7 @@ def gen_static_tu(st, ops, ctype: str, code: str) -> str:
             lines.append(
                 f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
                 f"&Shape_{name}::off[0][0], &launch_ymarch<{ctype}, {op}, Shape_{name}>, "
-                f"ymarch_gens<Elem<{ctype}>::raw>({L})}});")
+                f"ymarch_gens<Elem<{ctype}>::raw>({L}), 1}});")
             i += 1
     lines += ["}  // namespace", "}  // namespace sth", ""]
     return "\n".join(lines)

@@ -23,6 +23,7 @@
 #include "zmarch2_kernel.hpp"
 #include "zmarch1_kernel.hpp"
 #include "ymarch_kernel.hpp"
+#include "zmarch_kernel.hpp"
 #include "life2_kernel.hpp"
 #include "lifeb_kernel.hpp"
 #include "life_kernel.hpp"
@@ -630,23 +631,31 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
   apply_variant(pl, cands[0]);
   if (cands_out) *cands_out = std::move(cands);
 
-  // two steps per launch for 3-D radius-1 catalogue stencils (Wrap / Remove /
-  // Reflect)
-  // on arrays large enough for the z-marching kernel to beat two streaming
-  // steps: from 128^3 cells it measured 1.0-1.5x faster per step, from 256^3
-  // 1.5-2.8x (STH_FUSE3D_MIN_CELLS overrides the threshold)
+  // several steps per launch for 3-D radius-1 stencils (Wrap / Remove /
+  // Reflect): up to four for star stencils of 4-byte values, two
+  // (zmarch2_kernel) for the others on arrays large enough for it to beat two
+  // streaming steps: from 128^3 cells it measured 1.0-1.5x faster per step,
+  // from 256^3 1.5-2.8x (STH_FUSE3D_MIN_CELLS overrides the threshold)
   static const int64_t fuse3d_min = [] {
     const char* e = std::getenv("STH_FUSE3D_MIN_CELLS");
     return e ? std::atoll(e) : (int64_t(1) << 21);
   }();
   if (!pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 3 && st->ndim == 3 &&
       (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= 3 && n[1] >= 3 && n[2] >= 3 &&
-      n[0] * n[1] * n[2] >= fuse3d_min &&
       zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes && zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes) {
+    const bool big = cells >= fuse3d_min;
     for (const Fused2Entry* ep : catalogue(fused2_registry(), sdt, op->kind, L)) {
       const Fused2Entry& e = *ep;
-      if (e.ndim != st->ndim) continue;
-      if (!offsets_equal(e.offs, L, offs3)) continue;
+      if (e.ndim != st->ndim || !offsets_equal(e.offs, L, offs3)) continue;
+      if (e.any) {
+        if (!zmarch_pays(n[0], n[1], n[2], bc, dtype_size(sdt), kCus, big)) continue;
+        pl.fn_fused = e.fn;
+        pl.fused_gens = e.rows;
+        pl.fused_any = 1;
+        zmarch_grid(n[0], n[1], n[2], kCus, &pl.fused_tiles_x, &pl.fused_tiles_y, &pl.fused_tiles_z);
+        break;
+      }
+      if (!big) continue;
       static const int64_t zm_waves = [] {
         const char* v = std::getenv("STH_ZM2_WAVES");
         return v ? std::max<int64_t>(1, std::atoll(v)) : int64_t(8192);
@@ -657,7 +666,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       break;
     }
     // other radius-1 shapes and element types: the same kernel, runtime-compiled
-    if (!pl.fn_fused && sdt == odt && dtype_size(sdt) >= 2 && reach[0] <= 1 && reach[1] <= 1 && reach[2] <= 1 &&
+    if (!pl.fn_fused && big && sdt == odt && dtype_size(sdt) >= 2 && reach[0] <= 1 && reach[1] <= 1 && reach[2] <= 1 &&
         op->kind != STH_OP_LIFE && jit_wanted(n[0] * n[1] * n[2])) {
       std::vector<int8_t> o8(3 * static_cast<size_t>(L));
       for (size_t i = 0; i < o8.size(); ++i) o8[i] = static_cast<int8_t>(offs3[i]);

@@ -61,7 +61,8 @@ struct Fused2Entry {
   int ndim;
   const int8_t* offs;
   LaunchFn fn;
-  int rows;  // 3-D (two steps): rows per wave of the z-marching kernel; 2-D: most steps per launch
+  int rows;     // two steps (zmarch2_kernel): rows per wave; else most steps per launch
+  int any = 0;  // 1: the kernel takes any number of steps up to `rows`
 };
 std::vector<Fused2Entry>& fused2_registry();
 
