@@ -618,7 +618,7 @@ def bench_served(sh, torch, n: int = 120, budget: int = 2 << 30):
 
 def bench_heat_iterate(sh, torch, n: int = 512, steps: int = 200):
     """3-D heat iteration (VonNeumann(1,3) Laplacian(0.15), Wrap, n^3) as
-    `steps` hipGraph-replayed steps: two steps per launch (zmarch2_kernel)
+    `steps` hipGraph-replayed steps: several steps per launch (zmarch_kernel or zmarch2_kernel)
     against one streaming step per launch (STH_NO_FUSE).  The two-step
     kernel's roofline counts both steps' algorithmic bytes per launch."""
     f = sh.Laplacian(0.15)
@@ -706,7 +706,7 @@ def bench_heat3d_step(sh, torch, n: int = 512, reps: int = 10):
 
 def bench_heat_iterate_2d(sh, torch, steps: int = 100):
     """2-D heat iteration (VonNeumann(1) Laplacian(0.2), Wrap) as `steps`
-    hipGraph-replayed steps: two steps per launch (ymarch2_kernel) against one
+    hipGraph-replayed steps: several steps per launch (ymarch_kernel) against one
     streaming step per launch (STH_NO_FUSE); f32 and bf16 on 16384^2, f64 on
     8192^2 (a 16384^2 f64 grid is past the two-step kernel's 2 GiB offsets)."""
     f = sh.Laplacian(0.2)
@@ -734,7 +734,7 @@ def bench_heat_iterate_2d(sh, torch, steps: int = 100):
                      "two_step_achieved_gbs": 2 * 2 * es * n * n / (2 * t["two_step"] * 1e-6) / 1e9,
                      "one_step_achieved_gbs": 2 * es * n * n / (t["one_step"] * 1e-6) / 1e9}
         if name == "f32":
-            res[name]["two_step_traffic"] = profiled_traffic("ymarch2_kernel_heat2d_16384.md")
+            res[name]["two_step_traffic"] = None
         del A, S
         torch.cuda.empty_cache()
     return res
@@ -795,9 +795,8 @@ def main():
     S, wall, ev = time_steps(sh, torch, S, rule, args.steps, graph=True)
     bytes_per_step = 2 * cells  # 1 B read + 1 B written per interior cell and generation
     gen_us = ev / args.steps * 1e6
-    # The graph-replayed steady steps run lifeb_kernel: LIFE_GENS generations
-    # per launch (temporal blocking), so a launch's algorithmic bytes cover
-    # LIFE_GENS generations.  Its duration is timed on its own.
+    # The steady steps run lifep_kernel on packed bits (temporal blocking); the
+    # roofline is that of LIFE_GENS generations, timed on their own.
     S, launch_us = fused_launch_us(sh, torch, S, rule, LIFE_GENS)
     bytes_per_launch = LIFE_GENS * bytes_per_step
     achieved = bytes_per_launch / (launch_us * 1e-6) / 1e9
@@ -839,14 +838,13 @@ def main():
                                "launched directly below)", "cells": cells, "step": "one generation"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": profiled_traffic("lifeb_kernel_gol_8192.md"),
-                     "kernel": f"lifeb_kernel<G={LIFE_GENS}>: {LIFE_GENS} generations per launch, one bit "
+                     "traffic": None,
+                     "kernel": f"lifep_kernel: {LIFE_GENS} generations of it (a launch runs up to 32), one bit "
                                "per cell",
                      "bytes_per_launch": bytes_per_launch, "avg_launch_us": launch_us,
                      "per_generation_us": gen_us,
                      "note": "algorithmic bytes count 2 B per cell and generation (temporal-blocking "
-                             "savings excluded), so frac may exceed 1; traffic is the HBM bytes one "
-                             "launch moves (rocprofv3 FETCH_SIZE x2 + WRITE_SIZE)",
+                             "savings excluded), so frac may exceed 1",
                      "stream_copy_gbs": copy_gbs},
         "single_generation_kernel": {
             "kernel": "life_kernel<KY tuned, B3/S23>: one generation per launch (graph steps without temporal blocking)",
