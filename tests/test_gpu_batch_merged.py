@@ -37,3 +37,20 @@ def test_merged_batch(gpu, njobs, dtype):
     for i, (x, y) in enumerate(zip(calls, alone)):
         np.testing.assert_array_equal(x[1].float().cpu().numpy(), y[1].float().cpu().numpy(),
                                       err_msg=f"job {i}: {x[0]!r} {x[2]!r}")
+
+
+def test_large_batch_stays_apart(gpu):
+    """Variants of more than 8192 tiles on average keep a launch each."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(1)
+    calls, alone = [], []
+    for i in range(24):
+        a = torch.rand((1800, 2001), generator=g, device="cuda").T
+        f, st = (sh.sum, sh.Window(1)) if i % 2 else (sh.maximum, sh.Circle(3))
+        A = sh.StencilArray(a, st, boundary=sh.Wrap())
+        calls.append((f, sh.colmajor_empty((2001, 1800), torch.float32, "cuda"), A))
+        alone.append((f, sh.colmajor_empty((2001, 1800), torch.float32, "cuda"), A))
+    sh.BatchPlan(calls).run()
+    for (f, x, _), (_, y, A) in zip(calls, alone):
+        sh.mapstencil_(f, y, A)
+        assert torch.equal(x, y)
