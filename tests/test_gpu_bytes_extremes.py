@@ -31,3 +31,13 @@ def test_byte_extremes(gpu, oracle, size, bname, pad):
         ga, oa = (sh.StencilArray(A.copy(order="F"), st, boundary=bc, padding=padding) for _ in range(2))
         np.testing.assert_array_equal(sh.mapstencil(f, ga), oracle.mapstencil(f, oa), err_msg=repr(st))
     assert any("/bytes" in v for v in sh._lib.tuning_table().values())
+
+
+@pytest.mark.parametrize("bname", ["remove", "wrap", "reflect"])
+def test_byte_extremes_eight_rows(gpu, oracle, bname):
+    """From 2^25 cells a lane owns eight rows (reach up to 2)."""
+    rng = np.random.default_rng(7)
+    A = np.asfortranarray(rng.integers(0, 256, (8211, 4099)).astype(np.uint8))
+    bc = {"remove": sh.Remove(np.uint8(3)), "wrap": sh.Wrap(), "reflect": sh.Reflect()}[bname]
+    ga, oa = (sh.StencilArray(A, sh.Moore(2), boundary=bc) for _ in range(2))
+    np.testing.assert_array_equal(sh.mapstencil(sh.maximum, ga), oracle.mapstencil(sh.maximum, oa))
