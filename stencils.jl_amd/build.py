@@ -301,7 +301,8 @@ def gen_runtime_tu(ctype: str) -> str:
 # library's own, minus host-only and include flags.
 JIT_HEADERS = [("stencils_hip.h", REPO / "include" / "stencils_hip.h"), ("common.hpp", CSRC / "common.hpp"),
                ("tile_kernel.hpp", CSRC / "tile_kernel.hpp"), ("stream_kernel.hpp", CSRC / "stream_kernel.hpp"),
-               ("zmarch2_kernel.hpp", CSRC / "zmarch2_kernel.hpp"), ("ymarch_kernel.hpp", CSRC / "ymarch_kernel.hpp"),
+               ("zmarch2_kernel.hpp", CSRC / "zmarch2_kernel.hpp"), ("march_tiles.hpp", CSRC / "march_tiles.hpp"),
+               ("ymarch_kernel.hpp", CSRC / "ymarch_kernel.hpp"),
                ("scatter_kernel.hpp", CSRC / "scatter_kernel.hpp"), ("bytes_kernel.hpp", CSRC / "bytes_kernel.hpp")]
 JIT_OPTIONS = [f for f in CXXFLAGS if f not in ("-fPIC", "-Wno-unused-command-line-argument") and not f.startswith("-I")]
 

@@ -33,6 +33,7 @@
 
 #include <type_traits>
 
+#include "march_tiles.hpp"
 #include "stream_kernel.hpp"
 #include "tile_kernel.hpp"
 #include "zmarch2_kernel.hpp"
@@ -54,11 +55,6 @@ template <typename Raw>
 constexpr int ymarch_gens(int L) {
   return sizeof(Raw) == 2 ? 4 : (L <= 4 ? 8 : 6);
 }
-
-// Output lanes per wave: 56 lanes of 16 bytes make each row segment a whole
-// number of 128-byte lines (62 lanes measured 7% slower on 16384^2 f32 from
-// partial-line writes), and leave up to four rim lanes on each side.
-constexpr int kYmOut = 56;
 
 // Fewest cells per axis: more than the rims and a vector.
 constexpr int kYmMinCells = 16;
@@ -136,14 +132,9 @@ __global__ __launch_bounds__(256) void ymarch_kernel(MapParams p) {
   if (yb >= ye) return;  // uniform: the wave has no rows
   const int32_t gens = p.gens;      // generations of this launch, 1 .. G
   const int idle = G - gens;        // stages that pass rows on
-  // First output column.  Tiles of a row that is no whole number of vectors
-  // are spread evenly with the last one ending at the row's end, so that no
-  // lane's vector straddles either edge (cells of two tiles are computed and
-  // stored twice, with the same values).
-  const int32_t step = p.tiles_x > 1 ? (n0 - kYmOut * V) / (p.tiles_x - 1) : 0;
-  const bool spread = n0 % V != 0 && step >= RL * V;
-  const bool whole = n0 % V == 0 || spread;  // every vector lies wholly inside or outside the row (uniform)
-  const int32_t X0 = !spread ? bx * kYmOut * V : (bx == p.tiles_x - 1 ? n0 - kYmOut * V : bx * step);
+  const YmTiles tiles = ymarch_tiles(n0, p.tiles_x, V, RL);
+  const bool whole = n0 % V == 0 || tiles.spread;  // every vector lies wholly inside or outside the row (uniform)
+  const int32_t X0 = tiles.first(bx, V);            // first output column
   const Val pv = stage<S>(raw_from_bits<Raw>(p.padval));
   constexpr int64_t es = sizeof(Raw);
 
