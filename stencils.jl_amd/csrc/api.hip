@@ -271,9 +271,13 @@ const std::vector<const E*>& catalogue(const std::vector<E>& all, int dtype, int
   return it == index.end() ? none : it->second;
 }
 
+// The plan of one step from `src` to `dst`.  The kernels that advance several
+// steps per launch are chosen only for a caller that `iterates` with them:
+// one may have to be compiled first (a second or two), which a single gather
+// or a batch would wait for and never use.
 int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st, int32_t bc,
               const void* padval, int32_t padding, const sth_op* op, uint32_t flags, Plan* out,
-              std::vector<Variant>* cands_out = nullptr, std::string* group_out = nullptr) {
+              std::vector<Variant>* cands_out = nullptr, std::string* group_out = nullptr, bool iterates = false) {
   int rc;
   if ((rc = check_array(src, "source"))) return rc;
   if ((rc = check_array(dst, "dest"))) return rc;
@@ -642,7 +646,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
     const char* e = std::getenv("STH_FUSE3D_MIN_CELLS");
     return e ? std::atoll(e) : (int64_t(1) << 21);
   }();
-  if (!pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 3 && st->ndim == 3 &&
+  if (iterates && !pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 3 && st->ndim == 3 &&
       (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= 3 && n[1] >= 3 && n[2] >= 3 &&
       zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes && zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes) {
     const bool big = cells >= fuse3d_min;
@@ -699,7 +703,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
   auto rows4 = [](const DevArr& a, int64_t es) {
     return reinterpret_cast<uintptr_t>(a.base) % 4 == 0 && (a.s1 * es) % 4 == 0;
   };
-  if (!pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 2 && st->ndim == 2 &&
+  if (iterates && !pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 2 && st->ndim == 2 &&
       (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= kYmMinCells && n[1] >= kYmMinCells &&
       n[0] * n[1] >= fuse2d_min &&
       sdt == odt && rows4(pl.p.src, dtype_size(sdt)) && rows4(pl.p.dst, dtype_size(odt)) &&
@@ -1446,6 +1450,10 @@ int run_launches(sth_ctx* ctx, const Plan& ab, const Plan& ba, const char* kind,
                       [&](hipStream_t st) { return rest(st, reps * FU); });
 }
 
+// Fewest steps of which several may share a launch: with one launch for all
+// but the last step, three steps are no fewer launches than the steps are.
+constexpr int64_t kFuseMinSteps = 4;
+
 // Fewest steps of a Life iteration that run packed: pack, launches in pairs,
 // unpack and two single steps are then no more launches than the steps.
 constexpr int64_t kLifepMinSteps = 8;
@@ -2159,8 +2167,9 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
   Plan ab, ba;
   std::vector<Variant> cab, cba;
   std::string group;
-  if ((rc = make_plan(a, b, st, boundary, padval, padding, op, flags, &ab, &cab, &group))) return rc;
-  if ((rc = make_plan(b, a, st, boundary, padval, padding, op, flags, &ba, &cba))) return rc;
+  const bool iterates = steps >= kFuseMinSteps;
+  if ((rc = make_plan(a, b, st, boundary, padval, padding, op, flags, &ab, &cab, &group, iterates))) return rc;
+  if ((rc = make_plan(b, a, st, boundary, padval, padding, op, flags, &ba, &cba, nullptr, iterates))) return rc;
   auto s = static_cast<hipStream_t>(stream);
   if (steps > 0) {
     // choose the variant on the a -> b step (idempotent: it only writes b)
