@@ -654,11 +654,15 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       const Fused2Entry& e = *ep;
       if (e.ndim != st->ndim || !offsets_equal(e.offs, L, offs3)) continue;
       if (e.any) {
-        if (!zmarch_pays(n[0], n[1], n[2], bc, dtype_size(sdt), kCus, big)) continue;
+        if (n[0] < kZmMinCells || n[1] < kZmMinCells || n[2] < kZmMinCells) continue;
+        const ZmGrid grid = zmarch_grid(n[0], n[1], n[2], kCus);
+        if (!zmarch_pays(n[0], n[1], n[2], bc, dtype_size(sdt), grid, big)) continue;
         pl.fn_fused = e.fn;
         pl.fused_gens = e.rows;
         pl.fused_any = 1;
-        zmarch_grid(n[0], n[1], n[2], kCus, &pl.fused_tiles_x, &pl.fused_tiles_y, &pl.fused_tiles_z);
+        pl.fused_tiles_x = static_cast<int32_t>(grid.tx);
+        pl.fused_tiles_y = static_cast<int32_t>(grid.ty);
+        pl.fused_tiles_z = static_cast<int32_t>(grid.tz);
         break;
       }
       if (!big) continue;

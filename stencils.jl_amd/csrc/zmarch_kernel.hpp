@@ -32,17 +32,12 @@
 
 #include <type_traits>
 
+#include "march_tiles.hpp"
 #include "zmarch2_kernel.hpp"
 
 namespace sth {
 
-constexpr int kZmGens = 4;   // most steps per launch
-constexpr int kZmWaves = 8;  // two per SIMD: a wave takes up to 256 registers
-constexpr int kZmRows = 8;   // rows per wave
-constexpr int kZmOutX = 64 - 2 * kZmGens;
-constexpr int kZmOutY = kZmWaves * kZmRows - 2 * kZmGens;
 constexpr int kZmAhead = 3;  // planes loaded ahead
-constexpr int kZmMinCells = 16;  // fewest cells per axis: more than the rims
 
 // Offsets along one axis at a time, one cell: what the kernel's exchange covers.
 template <class Sh>
@@ -288,27 +283,6 @@ __global__ __launch_bounds__(64 * kZmWaves) void zmarch_kernel(MapParams p) {
   else march(std::integral_constant<int, kPlain>{});
 }
 
-// Grid of zmarch_kernel for an n0 x n1 x n2 array on `cus` compute units (a
-// workgroup fills one): the z chunks that make whole rounds shortest, a
-// workgroup's time being its planes and 2 G of overlap, in whole unrolled
-// groups of six.
-inline void zmarch_grid(int64_t n0, int64_t n1, int64_t n2, int cus, int32_t* tx, int32_t* ty, int32_t* tz) {
-  const int64_t gx = (n0 + kZmOutX - 1) / kZmOutX, gy = (n1 + kZmOutY - 1) / kZmOutY;
-  int64_t best = 1, least = 0;
-  for (int64_t c = 1; c <= n2; ++c) {
-    const int64_t zc = (n2 + c - 1) / c, chunks = (n2 + zc - 1) / zc;
-    if (chunks != c) continue;
-    const int64_t t = ((gx * gy * c + cus - 1) / cus) * ((zc + 2 * kZmGens + 5) / 6 * 6);
-    if (c == 1 || t < least) {
-      least = t;
-      best = c;
-    }
-  }
-  *tx = static_cast<int32_t>(gx);
-  *ty = static_cast<int32_t>(gy);
-  *tz = static_cast<int32_t>(best);
-}
-
 // Whether the kernel is the faster way to iterate an array: its time per step,
 // in us, against that of what would run otherwise.  Its own is the rounds of
 // workgroups times their plane steps, 0.35 us each and step (Wrap: 200^3 8.5,
@@ -318,14 +292,10 @@ inline void zmarch_grid(int64_t n0, int64_t n1, int64_t n2, int cus, int32_t* tx
 // 10.0, 256^3 17.5, 384^3 66, 512^3 162 us; 2-byte cells move half the bytes
 // and keep it); one launch per step below that 5 + 1.5 per 10^6 cells (32^3
 // 4.9, 100^3 7.9; here 3.9 and 4.5).
-inline bool zmarch_pays(int64_t n0, int64_t n1, int64_t n2, int bc, int es, int cus, bool zmarch2) {
-  if (n0 < kZmMinCells || n1 < kZmMinCells || n2 < kZmMinCells || (zmarch2 && es != 4)) return false;
-  int32_t tx, ty, tz;
-  zmarch_grid(n0, n1, n2, cus, &tx, &ty, &tz);
-  const int64_t steps = ((n2 + tz - 1) / tz + 2 * kZmGens + 5) / 6 * 6;
-  const int64_t rounds = (static_cast<int64_t>(tx) * ty * tz + cus - 1) / cus;
+inline bool zmarch_pays(int64_t n0, int64_t n1, int64_t n2, int bc, int es, const ZmGrid& grid, bool zmarch2) {
+  if (zmarch2 && es != 4) return false;
   const double here = (bc == STH_WRAP ? 0.35 : (bc == STH_REMOVE ? 0.47 : 0.5)) * (es == 4 ? 1.0 : 1.15) *
-                      static_cast<double>(rounds * steps);
+                      static_cast<double>(grid.time);
   const double mcells = 1e-6 * static_cast<double>(n0) * static_cast<double>(n1) * static_cast<double>(n2);
   const double other = zmarch2 ? (1.06 * mcells > 6.0 ? 1.06 * mcells : 6.0) : 5.0 + 1.5 * mcells;
   return here < other;

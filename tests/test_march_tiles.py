@@ -52,3 +52,56 @@ def run(tmp_path_factory):
 def test_column_tiles_cover_the_row(run):
     r = run(CHECK)
     assert r.returncode == 0, r.stdout
+
+
+ZGRID = r"""
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include "march_tiles.hpp"
+
+using sth::ZmGrid;
+
+// every chunk count that some chunk length gives, the first of the shortest
+static ZmGrid walk(int64_t n0, int64_t n1, int64_t n2, int64_t cus) {
+  const int64_t gx = (n0 + 55) / 56, gy = (n1 + 55) / 56;
+  ZmGrid best{gx, gy, 0, 0};
+  for (int64_t c = 1; c <= n2; ++c) {
+    const int64_t zc = (n2 + c - 1) / c;
+    if ((n2 + zc - 1) / zc != c) continue;
+    const int64_t t = (gx * gy * c + cus - 1) / cus * ((zc + 8 + 5) / 6 * 6);
+    if (best.tz == 0 || t < best.time) best = ZmGrid{gx, gy, c, t};
+  }
+  return best;
+}
+
+int main() {
+  int bad = 0;
+  auto one = [&](int64_t n0, int64_t n1, int64_t n2, int64_t cus) {
+    const ZmGrid a = sth::zmarch_grid(n0, n1, n2, cus), b = walk(n0, n1, n2, cus);
+    if ((a.tx != b.tx || a.ty != b.ty || a.tz != b.tz || a.time != b.time) && ++bad <= 5)
+      std::printf("%ld x %ld x %ld on %ld: %ld chunks, %ld, not %ld, %ld\n", long(n0), long(n1), long(n2), long(cus),
+                  long(a.tz), long(a.time), long(b.tz), long(b.time));
+  };
+  for (int64_t n2 = 16; n2 <= 1200; ++n2)
+    for (int64_t g = 1; g <= 40; ++g) one(g * 56 - 3, 50, n2, 256);
+  std::srand(1);
+  for (int i = 0; i < 20000; ++i)
+    one(16 + std::rand() % 2000, 16 + std::rand() % 2000, 16 + std::rand() % 3000, i % 3 ? 256 : 32 + std::rand() % 300);
+  one(16, 16, 1000000, 256);
+  one(3000, 300, 100000, 256);
+  long steps = 0;
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int64_t k = 0; k < 10; ++k) steps += sth::zmarch_grid(16, 16 + k, 1000000 + k, 256).tz;
+  const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() / 10;
+  std::printf("%d bad, %ld, %.2f us a search\n", bad, steps, us);
+  // (one search over 10^6 chunk counts takes milliseconds)
+  return bad != 0 || us > 200.0;
+}
+"""
+
+
+def test_plane_chunks_are_the_shortest(run):
+    r = run(ZGRID)
+    print(r.stdout)
+    assert r.returncode == 0, r.stdout
