@@ -168,6 +168,12 @@ int sth_version(void);
 /* Message of the last failed call on this thread ("" if none). */
 const char* sth_last_error(void);
 
+/* What the last sth_iterate of this thread ran its steps on: "single" (one
+ * launch per step) or a kernel that advances several per launch, with its
+ * most steps ("ymarch/8", "zmarch/4", "zmarch2/2", "lifep", ...).  For tests
+ * and measurements. */
+const char* sth_steps_kernel(void);
+
 /* Context: one per host thread.  `device` is a HIP device ordinal. */
 int sth_ctx_create(int device, sth_ctx** out);
 int sth_ctx_destroy(sth_ctx* ctx);

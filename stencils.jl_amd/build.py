@@ -162,21 +162,23 @@ def gen_static_tu(st, ops, ctype: str, code: str) -> str:
                 # up to four steps per launch (star stencils, 4-byte values)
                 lines.append(
                     f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
-                    f"&Shape_{name}::off[0][0], &launch_zmarch<{ctype}, {op}, Shape_{name}>, kZmGens, 1}});")
+                    f"&Shape_{name}::off[0][0], &launch_zmarch<{ctype}, {op}, Shape_{name}>, kZmGens, 1, "
+                    f"\"zmarch/4\"}});")
                 i += 1
             # two steps per launch for iterations (3-D: march along z)
             lines.append(
                 f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
                 f"&Shape_{name}::off[0][0], &launch_zmarch2<{ctype}, {op}, Shape_{name}>, "
-                f"zmarch2_rows<Staged<{ctype}>::type>()}});")
+                f"zmarch2_rows<Staged<{ctype}>::type>(), 0, \"zmarch2/2\"}});")
             i += 1
         if st.N == 2 and max(rx, ry) <= 1:
             # several steps per launch for iterations (2-D: march along y)
-            lines.append(
-                f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
-                f"&Shape_{name}::off[0][0], &launch_ymarch<{ctype}, {op}, Shape_{name}>, "
-                f"ymarch_gens<Elem<{ctype}>::raw>({L}), 1}});")
-            i += 1
+            for gens in (f"ymarch_gens<Elem<{ctype}>::raw>({L})", "kYmShortGens"):
+                lines.append(
+                    f"Registrar reg{i}(Fused2Entry{{{code}, {op}, {L}, {st.N}, "
+                    f"&Shape_{name}::off[0][0], &launch_ymarch<{ctype}, {op}, Shape_{name}, {gens}>, {gens}, 1, "
+                    f"ymarch_name({gens})}});")
+                i += 1
     lines += ["}  // namespace", "}  // namespace sth", ""]
     return "\n".join(lines)
 

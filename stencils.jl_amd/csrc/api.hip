@@ -20,6 +20,7 @@
 #include "bytes_kernel.hpp"
 #include "halo_kernel.hpp"
 #include "jit.hpp"
+#include "march_cost.hpp"
 #include "zmarch2_kernel.hpp"
 #include "zmarch1_kernel.hpp"
 #include "ymarch_kernel.hpp"
@@ -90,6 +91,7 @@ std::vector<BatchKernelEntry>& batch_kernels() {
 namespace {
 
 thread_local std::string g_err;
+thread_local const char* g_steps_kernel = "";  // sth_steps_kernel
 
 int fail(int code, const char* fmt, ...) {
   char buf[512];
@@ -154,6 +156,8 @@ struct Plan {
   int32_t jit_fused_3d;    // its grid: tiles_x * tiles_y (2-D) or * tiles_z (3-D)
   int32_t fused_gens;      // steps fn_fused advances per launch
   int32_t fused_any;       // it also advances any smaller number (MapParams::gens)
+  int64_t fused_singles;   // (fused_any) single steps at the end of the iteration planned for
+  const char* fused_name;  // "kernel/steps"
   int32_t fused_tiles_x, fused_tiles_y, fused_tiles_z;  // its grid
   int32_t life_packed;      // iterations may run on packed bits (lifep_kernel.hpp)
   HaloParams hp;
@@ -271,13 +275,24 @@ const std::vector<const E*>& catalogue(const std::vector<E>& all, int dtype, int
   return it == index.end() ? none : it->second;
 }
 
+// Calls of a few launches go straight to the stream even with STH_GRAPH: a
+// graph launch costs the host about 27 us against about 16 us for six direct
+// launches, and the device is the bound either way (Life 8192^2, 20 steps:
+// 152 us direct, 159 us replayed).
+constexpr int64_t kGraphMinLaunches = 17;
+
+// Fewest steps of which several may share a launch, where one single step
+// ends them: with one launch for the others, three steps are no fewer launches
+// than three.
+constexpr int64_t kFuseMinSteps = 4;
+
 // The plan of one step from `src` to `dst`.  The kernels that advance several
-// steps per launch are chosen only for a caller that `iterates` with them:
-// one may have to be compiled first (a second or two), which a single gather
-// or a batch would wait for and never use.
+// steps per launch are chosen only for a caller that runs `steps` steps with
+// it and its reverse: one may have to be compiled first (a second or two),
+// which a single gather or a batch would wait for and never use.
 int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st, int32_t bc,
               const void* padval, int32_t padding, const sth_op* op, uint32_t flags, Plan* out,
-              std::vector<Variant>* cands_out = nullptr, std::string* group_out = nullptr, bool iterates = false) {
+              std::vector<Variant>* cands_out = nullptr, std::string* group_out = nullptr, int64_t steps = 1) {
   int rc;
   if ((rc = check_array(src, "source"))) return rc;
   if ((rc = check_array(dst, "dest"))) return rc;
@@ -479,6 +494,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
                   : lg == 4 ? &launch_lifeb<4, 6, 0>
                             : (lnt ? &launch_lifeb<8, 6, 1> : &launch_lifeb<8, 6, 0>);
       pl.fused_gens = lg;
+      pl.fused_name = "lifeb";
       lifeb_grid(n[0], n[1], lg, lwaves, &pl.fused_tiles_x, &pl.fused_tiles_y);
       pl.fused_tiles_z = 1;
     } else if (vec16 && bc != STH_USE && n[1] >= 3) {
@@ -490,6 +506,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
                    : ky2 == 8 ? (conway ? &launch_life2<8, true> : &launch_life2<8, false>)
                               : (conway ? &launch_life2<4, true> : &launch_life2<4, false>);
       pl.fused_gens = 2;
+      pl.fused_name = "life2";
       pl.fused_tiles_x = static_cast<int32_t>((n[0] + 1023) / 1024);
       pl.fused_tiles_y = static_cast<int32_t>((n[1] + 4 * ky2 - 1) / (4 * ky2));
       pl.fused_tiles_z = 1;
@@ -637,56 +654,75 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
   apply_variant(pl, cands[0]);
   if (cands_out) *cands_out = std::move(cands);
 
-  // several steps per launch for 3-D radius-1 stencils (Wrap / Remove /
-  // Reflect): up to four for star stencils of 4-byte values, two
-  // (zmarch2_kernel) for the others on arrays large enough for it to beat two
-  // streaming steps: from 128^3 cells it measured 1.0-1.5x faster per step,
-  // from 256^3 1.5-2.8x (STH_FUSE3D_MIN_CELLS overrides the threshold)
+  // Several steps per launch (Wrap / Remove / Reflect; radius 1).  Every
+  // iteration ends with a single step, with a halo two (each refreshes its
+  // source's halo).  STH_STEPS_KERNEL, read per call, names the kernel to use
+  // wherever it can run ("zmarch/4", "zmarch2/2", "ymarch/8", "ymarch/2", ...,
+  // "single"), to test and compare them.
+  const int64_t least_singles = halo_pad && src->halo > 0 ? 2 : 1;
+  const bool multi = steps >= kFuseMinSteps + least_singles - 1 && !pl.fn_fused &&
+                     !(flags & (STH_NO_FUSE | STH_GENERIC)) &&
+                     (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) &&
+                     zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes &&
+                     zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes;
+  const char* const wanted = multi ? std::getenv("STH_STEPS_KERNEL") : nullptr;
+
+  // 3-D: up to four steps for star stencils of 4-byte values (zmarch_kernel),
+  // two (zmarch2_kernel) for the others on arrays large enough for it to beat
+  // two streaming steps: from 128^3 cells it measured 1.0-1.5x faster per
+  // step, from 256^3 1.5-2.8x (STH_FUSE3D_MIN_CELLS overrides the threshold)
   static const int64_t fuse3d_min = [] {
     const char* e = std::getenv("STH_FUSE3D_MIN_CELLS");
     return e ? std::atoll(e) : (int64_t(1) << 21);
   }();
-  if (iterates && !pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 3 && st->ndim == 3 &&
-      (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= 3 && n[1] >= 3 && n[2] >= 3 &&
-      zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes && zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes) {
+  if (multi && src->ndim == 3 && st->ndim == 3 && n[0] >= 3 && n[1] >= 3 && n[2] >= 3) {
     const bool big = cells >= fuse3d_min;
     for (const Fused2Entry* ep : catalogue(fused2_registry(), sdt, op->kind, L)) {
       const Fused2Entry& e = *ep;
       if (e.ndim != st->ndim || !offsets_equal(e.offs, L, offs3)) continue;
+      if (wanted && std::strcmp(wanted, e.name) != 0) continue;
       if (e.any) {
         if (n[0] < kZmMinCells || n[1] < kZmMinCells || n[2] < kZmMinCells) continue;
         const ZmGrid grid = zmarch_grid(n[0], n[1], n[2], kCus);
-        if (!zmarch_pays(n[0], n[1], n[2], bc, dtype_size(sdt), grid, big)) continue;
+        const int64_t singles =
+            wanted ? least_singles
+                   : zmarch_singles(n[0], n[1], n[2], bc, dtype_size(sdt), grid, big, least_singles > 1,
+                                    (flags & STH_GRAPH) != 0 && steps >= kGraphMinLaunches, steps, least_singles);
+        if (singles >= steps) continue;
         pl.fn_fused = e.fn;
         pl.fused_gens = e.rows;
         pl.fused_any = 1;
+        pl.fused_singles = singles;
+        pl.fused_name = e.name;
         pl.fused_tiles_x = static_cast<int32_t>(grid.tx);
         pl.fused_tiles_y = static_cast<int32_t>(grid.ty);
         pl.fused_tiles_z = static_cast<int32_t>(grid.tz);
         break;
       }
-      if (!big) continue;
+      if (!big && !wanted) continue;
       static const int64_t zm_waves = [] {
         const char* v = std::getenv("STH_ZM2_WAVES");
         return v ? std::max<int64_t>(1, std::atoll(v)) : int64_t(8192);
       }();
       pl.fn_fused = e.fn;
       pl.fused_gens = 2;
+      pl.fused_name = e.name;
       zmarch2_grid(n[0], n[1], n[2], e.rows, zm_waves, &pl.fused_tiles_x, &pl.fused_tiles_y, &pl.fused_tiles_z);
       break;
     }
     // other radius-1 shapes and element types: the same kernel, runtime-compiled
-    if (!pl.fn_fused && big && sdt == odt && dtype_size(sdt) >= 2 && reach[0] <= 1 && reach[1] <= 1 && reach[2] <= 1 &&
+    if (!pl.fn_fused && (wanted ? std::strcmp(wanted, "zmarch2/2") == 0 : big) && sdt == odt && dtype_size(sdt) >= 2 && reach[0] <= 1 && reach[1] <= 1 && reach[2] <= 1 &&
         op->kind != STH_OP_LIFE && jit_wanted(n[0] * n[1] * n[2])) {
       std::vector<int8_t> o8(3 * static_cast<size_t>(L));
       for (size_t i = 0; i < o8.size(); ++i) o8[i] = static_cast<int8_t>(offs3[i]);
       std::string why;
-      if (const JitKernel* jk = jit_fused_kernel(sdt, op->kind, L, o8.data(), 1, 1, 1, 3, bc, &why)) {
+      if (const JitKernel* jk = jit_fused_kernel(sdt, op->kind, L, o8.data(), 1, 1, 1, 3, bc, 2, &why)) {
         const char* v = std::getenv("STH_ZM2_WAVES");
         const int64_t zw = v ? std::max<int64_t>(1, std::atoll(v)) : int64_t(8192);
         pl.jit_fused = jk->fn;
         pl.jit_fused_3d = 1;
         pl.fused_gens = 2;
+        pl.fused_name = "zmarch2/2";
         zmarch2_grid(n[0], n[1], n[2], jit_zmarch2_rows(sdt), zw, &pl.fused_tiles_x, &pl.fused_tiles_y,
                      &pl.fused_tiles_z);
       } else {
@@ -695,48 +731,58 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
     }
   }
 
-  // several steps per launch for 2-D radius-1 stencils (Wrap / Remove /
-  // Reflect) on arrays whose rows start on 4-byte boundaries (vectors are
-  // 16-byte buffer accesses at any such offset), of any size: 64^2 f32 heat
-  // takes 1.4 us per step against 2.7 with one launch per step
-  // (STH_FUSE2D_MIN_CELLS sets a smallest size)
+  // 2-D: rows that start on 4-byte boundaries (vectors are 16-byte buffer
+  // accesses at any such offset), of any size: 64^2 f32 heat takes 1.4 us per
+  // step against 2.7 with one launch per step.  Long launches, short ones or
+  // single steps as march_choose has it; with STH_FUSE2D_MIN_CELLS long ones
+  // for every array of so many cells, and none below.
   static const int64_t fuse2d_min = [] {
     const char* e = std::getenv("STH_FUSE2D_MIN_CELLS");
-    return e ? std::atoll(e) : int64_t(0);
+    return e ? std::atoll(e) : int64_t(-1);
   }();
-  auto rows4 = [](const DevArr& a, int64_t es) {
-    return reinterpret_cast<uintptr_t>(a.base) % 4 == 0 && (a.s1 * es) % 4 == 0;
+  auto rows_on = [](const DevArr& a, int64_t es, int64_t bytes) {
+    return reinterpret_cast<uintptr_t>(a.base) % bytes == 0 && (a.s1 * es) % bytes == 0;
   };
-  if (iterates && !pl.fn_fused && !(flags & (STH_NO_FUSE | STH_GENERIC)) && src->ndim == 2 && st->ndim == 2 &&
-      (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) && n[0] >= kYmMinCells && n[1] >= kYmMinCells &&
-      n[0] * n[1] >= fuse2d_min &&
-      sdt == odt && rows4(pl.p.src, dtype_size(sdt)) && rows4(pl.p.dst, dtype_size(odt)) &&
-      zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes && zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes) {
-    for (const Fused2Entry* ep : catalogue(fused2_registry(), sdt, op->kind, L)) {
-      const Fused2Entry& e = *ep;
-      if (e.ndim != 2) continue;
-      if (!offsets_equal(e.offs, L, offs3)) continue;
-      pl.fn_fused = e.fn;
-      pl.fused_gens = e.rows;
-      break;
-    }
-    if (!pl.fn_fused && dtype_size(sdt) >= 2 && reach[0] <= 1 && reach[1] <= 1 && op->kind != STH_OP_LIFE &&
-        jit_wanted(n[0] * n[1])) {
-      std::vector<int8_t> o8(3 * static_cast<size_t>(L));
-      for (size_t i = 0; i < o8.size(); ++i) o8[i] = static_cast<int8_t>(offs3[i]);
-      std::string why;
-      if (const JitKernel* jk = jit_fused_kernel(sdt, op->kind, L, o8.data(), 1, 1, 0, 2, bc, &why)) {
-        pl.jit_fused = jk->fn;
-        pl.jit_fused_3d = 0;
-        pl.fused_gens = jit_ymarch_gens(sdt, L);
-      } else {
-        jit_note("multi-step 2-D kernel", why);
+  const int64_t es2 = dtype_size(sdt);
+  if (multi && src->ndim == 2 && st->ndim == 2 && n[0] >= kYmMinCells && n[1] > kYmShortGens && cells >= fuse2d_min &&
+      sdt == odt && reach[0] <= 1 && reach[1] <= 1 && rows_on(pl.p.src, es2, 4) && rows_on(pl.p.dst, es2, 4)) {
+    const Fused2Entry* built[2] = {};  // long launches, short ones
+    for (const Fused2Entry* e : catalogue(fused2_registry(), sdt, op->kind, L))
+      if (e->ndim == 2 && offsets_equal(e->offs, L, offs3)) built[e->rows == kYmShortGens] = e;
+    const bool compiled = !built[0] && es2 >= 2 && op->kind != STH_OP_LIFE && jit_wanted(cells);
+    if (built[0] || compiled) {
+      const int most = built[0] ? built[0]->rows : jit_ymarch_gens(sdt, L);
+      MarchChoice c{n[1] >= kYmMinCells ? most : 0, least_singles};
+      if (wanted) {
+        c.gens = std::strcmp(wanted, ymarch_name(kYmShortGens)) == 0         ? kYmShortGens
+                 : c.gens && std::strcmp(wanted, ymarch_name(most)) == 0 ? most
+                                                                             : 0;
+      } else if (fuse2d_min < 0) {
+        const MarchCall call{n[0], n[1], sdt, op->kind, L, bc,
+                             rows_on(pl.p.src, es2, 16) && rows_on(pl.p.dst, es2, 16), built[0] != nullptr, least_singles > 1};
+        c = march_choose(call, most, steps, least_singles, kCus);
       }
-    }
-    if (pl.fn_fused || pl.jit_fused) {
-      pl.fused_any = 1;
-      ymarch_grid(n[0], n[1], 16 / dtype_size(sdt), pl.fused_gens, kCus, &pl.fused_tiles_x, &pl.fused_tiles_y,
-                  &pl.fused_tiles_z);
+      if (c.gens && built[0]) {
+        pl.fn_fused = built[c.gens == kYmShortGens]->fn;
+      } else if (c.gens) {
+        std::vector<int8_t> o8(3 * static_cast<size_t>(L));
+        for (size_t i = 0; i < o8.size(); ++i) o8[i] = static_cast<int8_t>(offs3[i]);
+        std::string why;
+        if (const JitKernel* jk = jit_fused_kernel(sdt, op->kind, L, o8.data(), 1, 1, 0, 2, bc, c.gens, &why))
+          pl.jit_fused = jk->fn;
+        else
+          jit_note("multi-step 2-D kernel", why);
+      }
+      if (pl.fn_fused || pl.jit_fused) {
+        pl.fused_gens = c.gens;
+        pl.fused_any = 1;
+        pl.fused_singles = c.singles;
+        pl.fused_name = ymarch_name(c.gens);
+        const YmGrid grid = ymarch_grid(n[0], n[1], static_cast<int>(16 / es2), c.gens, kCus);
+        pl.fused_tiles_x = static_cast<int32_t>(grid.tx);
+        pl.fused_tiles_y = static_cast<int32_t>(grid.ty);
+        pl.fused_tiles_z = static_cast<int32_t>(grid.rows);
+      }
     }
   }
 
@@ -1361,12 +1407,6 @@ static int clear_graphs(sth_ctx* ctx) {
 }
 
 namespace {
-// Calls of a few launches go straight to the stream even with STH_GRAPH: a
-// graph launch costs the host about 27 us against about 16 us for six direct
-// launches, and the device is the bound either way (Life 8192^2, 20 steps:
-// 152 us direct, 159 us replayed).
-constexpr int64_t kGraphMinLaunches = 17;
-
 // Launches the graph that `enqueue(stream)` records, `times` times on `s`.
 // Graphs of an iteration's steps are captured once per parameter set (the
 // bytes of its two step plans, and `tag`: the step layout) and replayed.  The
@@ -1410,22 +1450,18 @@ int replay_graph(sth_ctx* ctx, const Plan& ab, const Plan& ba, const std::string
   return STH_OK;
 }
 
-// `gens` steps as launches of at most G steps each, the smallest number F of
-// launches that has the parity of `gens` (so the buffers alternate as step by
-// step): all take G steps but the last four, which share the rest.  Calls
+// `gens` steps as march_launches of at most G steps each, by march_share.  Calls
 // head(stream), advance(stream, i, steps of launch i) and finish(stream, F);
 // with STH_GRAPH and enough launches 32 full launches are one graph,
 // replayed, and the rest of the call another (`kind` names the caller).
 template <class Head, class Advance, class Finish>
 int run_launches(sth_ctx* ctx, const Plan& ab, const Plan& ba, const char* kind, int64_t gens, int64_t G, uint32_t flags,
                  hipStream_t s, Head&& head, Advance&& advance, Finish&& finish) {
-  int64_t F = (gens + G - 1) / G;
-  if ((F ^ gens) & 1) ++F;
-  const int64_t full = std::max<int64_t>(0, F - 4);
+  const int64_t F = march_launches(gens, G), full = std::max<int64_t>(0, F - 4);
   auto rest = [&](hipStream_t st, int64_t from) -> int {
     int64_t left = gens - from * G;
     for (int64_t i = from; i < F; ++i) {
-      const int64_t g = i < full ? G : (left + (F - i) - 1) / (F - i);
+      const int64_t g = march_share(i, F, left, G);
       left -= g;
       if (int rc = advance(st, i, g)) return rc;
     }
@@ -1453,10 +1489,6 @@ int run_launches(sth_ctx* ctx, const Plan& ab, const Plan& ba, const char* kind,
   return replay_graph(ctx, ab, ba, tag('r', gens - reps * FU * G), 1, s,
                       [&](hipStream_t st) { return rest(st, reps * FU); });
 }
-
-// Fewest steps of which several may share a launch: with one launch for all
-// but the last step, three steps are no fewer launches than the steps are.
-constexpr int64_t kFuseMinSteps = 4;
 
 // Fewest steps of a Life iteration that run packed: pack, launches in pairs,
 // unpack and two single steps are then no more launches than the steps.
@@ -1521,6 +1553,8 @@ extern "C" {
 int sth_version(void) { return STH_ABI_VERSION * 10000 + 0; }
 
 const char* sth_last_error(void) { return g_err.c_str(); }
+
+const char* sth_steps_kernel(void) { return g_steps_kernel; }
 
 int sth_ctx_create(int device, sth_ctx** out) {
   STH_GUARD_BEGIN
@@ -2171,9 +2205,8 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
   Plan ab, ba;
   std::vector<Variant> cab, cba;
   std::string group;
-  const bool iterates = steps >= kFuseMinSteps;
-  if ((rc = make_plan(a, b, st, boundary, padval, padding, op, flags, &ab, &cab, &group, iterates))) return rc;
-  if ((rc = make_plan(b, a, st, boundary, padval, padding, op, flags, &ba, &cba, nullptr, iterates))) return rc;
+  if ((rc = make_plan(a, b, st, boundary, padval, padding, op, flags, &ab, &cab, &group, steps))) return rc;
+  if ((rc = make_plan(b, a, st, boundary, padval, padding, op, flags, &ba, &cba, nullptr, steps))) return rc;
   auto s = static_cast<hipStream_t>(stream);
   if (steps > 0) {
     // choose the variant on the a -> b step (idempotent: it only writes b)
@@ -2184,7 +2217,9 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
   }
   *current = static_cast<int32_t>(steps % 2);
   if (steps == 0) return STH_OK;
+  g_steps_kernel = "single";
   if (ab.life_packed && steps >= kLifepMinSteps) {
+    g_steps_kernel = "lifep";
     if ((rc = iterate_life_packed(ctx, ab, ba, steps, flags, s))) return rc;
     if (!(flags & STH_ASYNC)) STH_HIP(hipStreamSynchronize(s));
     return STH_OK;
@@ -2194,8 +2229,9 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
     // interiors and the newest generation, so the last step is a single one
     // (the other buffer then holds the step before), and with a halo the
     // last two (each refreshes its source's halo).
-    const int64_t single = ab.halo ? 2 : 1, gens = steps - single;
-    if (gens > 0 && (gens + ab.fused_gens - 1) / ab.fused_gens + 1 + single < steps) {
+    const int64_t single = ab.fused_singles, gens = steps - single;
+    if (gens > 0 && march_launches(gens, ab.fused_gens) + single < steps) {
+      g_steps_kernel = ab.fused_name;
       if ((rc = run_launches(
                ctx, ab, ba, "flex", gens, ab.fused_gens, flags, s, [](hipStream_t) { return STH_OK; },
                [&](hipStream_t st, int64_t i, int64_t g) { return run_fused(i % 2 ? ba : ab, st, g); },
@@ -2223,6 +2259,7 @@ int sth_iterate(sth_ctx* ctx, const sth_array* a, const sth_array* b, const sth_
   const int64_t G = ab.fused_gens;
   const bool fuse = !(flags & STH_NO_FUSE) && (ab.fn_fused || ab.jit_fused) && (ba.fn_fused || ba.jit_fused) &&
                     !ab.fused_any && !ba.fused_any && G >= 2 && rest >= 2 * G + 2;
+  if (fuse) g_steps_kernel = ab.fused_name;
   const int64_t units = fuse ? (rest - 2) / (2 * G) : 0;  // fused pairs
   const int64_t tail = rest - 2 * G * units;              // single steps (2 .. 2G + 1 when fused)
   auto enqueue = [&](hipStream_t st, bool first, int64_t nunits, int64_t nplain) -> int {
@@ -2473,7 +2510,7 @@ int sth_jit_selftest(char* log, size_t cap) {
   for (const auto& c : fdt) {
     std::string src, expr;
     jit_fused_source(c[0], c[1], c[2] == 3 ? 6 : 4, c[2] == 3 ? &vn3[0][0] : &vn2[0][0], 1, 1, c[2] == 3 ? 1 : 0, c[2],
-                     STH_WRAP, &src, &expr);
+                     STH_WRAP, 2, &src, &expr);
     one(src, expr, std::string("two-step ") + std::to_string(c[2]) + "-D " + jit_type_name(c[0]));
   }
   {

@@ -645,12 +645,12 @@ inline int jit_ymarch_gens(int dtype, int L) {
 // radius-1 shape: ymarch_kernel (2-D) or zmarch2_kernel (3-D) for
 // boundary `bc` (false: no type name).
 inline bool jit_fused_source(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz, int ndim, int bc,
-                             std::string* src_out, std::string* expr_out) {
+                             int gens, std::string* src_out, std::string* expr_out) {
   const char* tn = jit_type_name(dtype);
   if (!tn) return false;
   const std::string head = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, ";
   const std::string targs = ndim == 3 ? head + std::to_string(jit_zmarch2_rows(dtype)) + ", " + std::to_string(bc)
-                                      : head + std::to_string(jit_ymarch_gens(dtype, L)) + ", " + std::to_string(bc);
+                                      : head + std::to_string(gens) + ", " + std::to_string(bc);
   const std::string kern = ndim == 3 ? "zmarch2_kernel" : "ymarch_kernel";
   *src_out = "#include \"ymarch_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, rz) +
              "namespace sth {\ntemplate __global__ void " + kern + "<" + targs + ">(MapParams);\n}  // namespace sth\n";
@@ -659,11 +659,12 @@ inline bool jit_fused_source(int dtype, int opk, int L, const int8_t* offs3, int
 }
 
 inline const JitKernel* jit_fused_kernel(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz,
-                                         int ndim, int bc, std::string* why) {
-  const JitRequest request = JitRequest('f').add(dtype).add(opk).add(rx).add(ry).add(rz).add(ndim).add(bc).add(offs3, 3 * static_cast<size_t>(L));
+                                         int ndim, int bc, int gens, std::string* why) {
+  const JitRequest request = JitRequest('f').add(dtype).add(opk).add(rx).add(ry).add(rz)
+                                 .add(ndim).add(bc).add(gens).add(offs3, 3 * static_cast<size_t>(L));
   return jit_remembered(request, [&]() -> const JitKernel* {
     std::string src, expr;
-    if (!jit_fused_source(dtype, opk, L, offs3, rx, ry, rz, ndim, bc, &src, &expr)) {
+    if (!jit_fused_source(dtype, opk, L, offs3, rx, ry, rz, ndim, bc, gens, &src, &expr)) {
       *why = "no type name";
       return nullptr;
     }

@@ -35,6 +35,61 @@ constexpr YmTiles ymarch_tiles(int n0, int tiles, int v, int rim) {
   return YmTiles{step, tiles > 1 ? slack - step * (tiles - 1) : 0, n0 % v != 0 && step >= rim * v};
 }
 
+// Fewest steps per launch that ymarch_kernel is built for.
+constexpr int kYmShortGens = 2;
+
+// Fewest cells per axis: more than the rims and a vector.
+constexpr int kYmMinCells = 16;
+
+// Rows loaded ahead of the row consumed: two workgroups per CU (the
+// registers' limit) need six.  4096^2 f32, 8 generations: 6.9 us per step with
+// three rows ahead, 5.3 with six.
+constexpr int kYmAhead = 6;
+
+// The name of ymarch_kernel built for `gens` steps per launch.
+constexpr const char* ymarch_name(int gens) {
+  return gens == 8 ? "ymarch/8" : gens == 6 ? "ymarch/6" : gens == 4 ? "ymarch/4" : "ymarch/2";
+}
+
+struct YmGrid {
+  int64_t tx, ty, rows;  // column tiles, groups of four row chunks, rows per chunk
+};
+
+// Grid of ymarch_kernel for an n0 x n1 array: 56 V-column tiles x groups of
+// four row chunks; the chunk length travels in tiles_z.  A wave's time is
+// rows + 2 G row steps, each about w + 1/4 of a wave's issue time on a CU
+// that holds w workgroups (and no less than 1.6 of it alone, where latency
+// shows), so one or two workgroups per CU, or a few rounds of two, are
+// compared: 4096^2 f32, 8 generations: one per CU 64 us, two 48 us, three
+// 50 us; a partial second round costs a whole one.
+constexpr YmGrid ymarch_grid(int64_t n0, int64_t n1, int v, int gens, int64_t cus) {
+  const int64_t gx = (n0 + kYmOut * v - 1) / (kYmOut * v);
+  if (gens == kYmShortGens) {  // bound by memory: as many waves as fill every SIMD several times over
+    const int64_t chunks = (32 * cus + gx - 1) / gx;
+    int64_t rc = (n1 + chunks - 1) / chunks;
+    if (rc < 14) rc = 14;
+    rc = (rc + 2 * gens + kYmAhead - 1) / kYmAhead * kYmAhead - 2 * gens;
+    return YmGrid{gx, (n1 + 4 * rc - 1) / (4 * rc), rc};
+  }
+  int64_t best_rc = n1;
+  double least = 0;
+  for (int c = 0; c < 6; ++c) {  // one workgroup per CU, then 1 .. 5 rounds of two
+    const int64_t blocks = c == 0 ? cus : 2 * cus * c;
+    const int64_t g = blocks / gx > 0 ? blocks / gx : 1;
+    // row steps come in whole unrolled groups
+    const int64_t steps = ((n1 + 4 * g - 1) / (4 * g) + 2 * gens + kYmAhead - 1) / kYmAhead * kYmAhead;
+    const int64_t rc = steps - 2 * gens;
+    const int64_t total = gx * ((n1 + 4 * rc - 1) / (4 * rc));
+    const double rounds = static_cast<double>((total + 2 * cus - 1) / (2 * cus));
+    const double t = static_cast<double>(steps) * (total <= cus ? 1.6 : 2.25 * rounds);
+    if (c == 0 || t < least) {
+      least = t;
+      best_rc = rc;
+    }
+  }
+  return YmGrid{gx, (n1 + 4 * best_rc - 1) / (4 * best_rc), best_rc};
+}
+
 constexpr int kZmGens = 4;   // most steps per launch of zmarch_kernel
 constexpr int kZmWaves = 8;  // two per SIMD: a wave takes up to 256 registers
 constexpr int kZmRows = 8;   // rows per wave

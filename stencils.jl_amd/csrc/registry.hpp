@@ -62,7 +62,8 @@ struct Fused2Entry {
   const int8_t* offs;
   LaunchFn fn;
   int rows;     // two steps (zmarch2_kernel): rows per wave; else most steps per launch
-  int any = 0;  // 1: the kernel takes any number of steps up to `rows`
+  int any;      // 1: the kernel takes any number of steps up to `rows`
+  const char* name;
 };
 std::vector<Fused2Entry>& fused2_registry();
 

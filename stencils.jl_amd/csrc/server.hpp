@@ -168,7 +168,7 @@ struct sth_server {
         std::vector<sth::Variant> cands;
         std::string group;
         prc = sth::make_plan(c ? &b : &a, c ? &a : &b, &st, q.r.boundary, &q.padval, q.r.padding, &q.r.op, 0,
-                             &q.plan[c], &cands, &group, q.cells >= solo_cells());
+                             &q.plan[c], &cands, &group, q.cells >= solo_cells() ? q.r.steps : 1);
         int idx = 0;
         if (prc == STH_OK) prc = tune_pick(ctx, q.plan[c], cands, group, 0, stream, false, true, &idx);
         if (prc == STH_OK) sth::apply_variant(q.plan[c], cands[idx]);

@@ -20,7 +20,9 @@
 //
 // What bounds it: vector operations and their latency (the bytes of 4096^2
 // f32, 8 steps per launch, take 3 us per step).  100 steps of f32 heat on
-// 4096^2: 1675 us with two steps per launch, 636 us now.
+// 4096^2: 1675 us with two steps per launch, 636 us with eight.  Where the rims
+// are most of what eight (six, four) steps compute, the host launches the
+// kernel built for two (march_cost.hpp).
 //
 // Exactness: every value uses the shared fold expressions in offset order,
 // every generation is rounded to the storage type as a store would round it,
@@ -55,14 +57,6 @@ template <typename Raw>
 constexpr int ymarch_gens(int L) {
   return sizeof(Raw) == 2 ? 4 : (L <= 4 ? 8 : 6);
 }
-
-// Fewest cells per axis: more than the rims and a vector.
-constexpr int kYmMinCells = 16;
-
-// Rows loaded ahead of the row consumed: two workgroups per CU (the
-// registers' limit) need six.  4096^2 f32, 8 generations: 6.9 us per step with
-// three rows ahead, 5.3 with six.
-constexpr int kYmAhead = 6;
 
 // One fold over the stencil at element i of a lane's vector: row slots q0
 // (dy = -1), q1, q2; lm / rp are the element left of element 0 and right of
@@ -147,8 +141,8 @@ __global__ __launch_bounds__(256) void ymarch_kernel(MapParams p) {
   constexpr uint32_t kDrop = 0x80000000u;
 
   // mapped coordinate of c; cells beyond the G-cell rim feed no stored
-  // result and are clamped into it first (n >= kYmMinCells > G, checked on the
-  // host, so every mapped rim cell lies inside the array)
+  // result and are clamped into it first (n >= kYmMinCells > G, or n > G = 2
+  // rows, checked on the host, so every mapped rim cell lies inside the array)
   auto map_c = [&](int32_t c, int32_t n) -> int32_t {
     c = c < -G ? -G : (c > n + G - 1 ? n + G - 1 : c);
     if (c < 0) return REMOVE ? 0 : (REFLECT ? -c : c + n);
@@ -390,39 +384,8 @@ __global__ __launch_bounds__(256) void ymarch_kernel(MapParams p) {
     march(std::integral_constant<int, kPlain>{});
 }
 
-// Grid of ymarch_kernel for an n0 x n1 array: 56 V-column tiles x groups of
-// four row chunks; the chunk length travels in tiles_z.  A wave's time is
-// rows + 2 G row steps, each about w + 1/4 of a wave's issue time on a CU
-// that holds w workgroups (and no less than 1.6 of it alone, where latency
-// shows), so one or two workgroups per CU, or a few rounds of two, are
-// compared: 4096^2 f32, 8 generations: one per CU 64 us, two 48 us, three
-// 50 us; a partial second round costs a whole one.
-inline void ymarch_grid(int64_t n0, int64_t n1, int v, int gens, int cus, int32_t* tx, int32_t* ty, int32_t* rows) {
-  const int64_t gx = (n0 + kYmOut * v - 1) / (kYmOut * v);
-  int64_t best_rc = n1;
-  double least = 0;
-  for (int c = 0; c < 6; ++c) {  // one workgroup per CU, then 1 .. 5 rounds of two
-    const int64_t blocks = c == 0 ? cus : 2 * int64_t(cus) * c;
-    const int64_t g = blocks / gx > 0 ? blocks / gx : 1;
-    // row steps come in whole unrolled groups
-    const int64_t steps = ((n1 + 4 * g - 1) / (4 * g) + 2 * gens + kYmAhead - 1) / kYmAhead * kYmAhead;
-    const int64_t rc = steps - 2 * gens;
-    const int64_t total = gx * ((n1 + 4 * rc - 1) / (4 * rc));
-    const double rounds = static_cast<double>((total + 2 * cus - 1) / (2 * cus));
-    const double t = static_cast<double>(steps) * (total <= cus ? 1.6 : 2.25 * rounds);
-    if (c == 0 || t < least) {
-      least = t;
-      best_rc = rc;
-    }
-  }
-  *tx = static_cast<int32_t>(gx);
-  *ty = static_cast<int32_t>((n1 + 4 * best_rc - 1) / (4 * best_rc));
-  *rows = static_cast<int32_t>(best_rc);
-}
-
-template <typename S, int OPK, class Sh>
+template <typename S, int OPK, class Sh, int G>
 void launch_ymarch(const MapParams& p, hipStream_t s) {
-  constexpr int G = ymarch_gens<typename Elem<S>::raw>(Sh::L);
   const unsigned nb = static_cast<unsigned>(p.tiles_x) * p.tiles_y;
   if (p.bc == STH_REMOVE)
     hipLaunchKernelGGL((ymarch_kernel<S, OPK, Sh, G, STH_REMOVE>), dim3(nb), dim3(256), 0, s, p);

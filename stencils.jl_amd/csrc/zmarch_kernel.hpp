@@ -283,24 +283,6 @@ __global__ __launch_bounds__(64 * kZmWaves) void zmarch_kernel(MapParams p) {
   else march(std::integral_constant<int, kPlain>{});
 }
 
-// Whether the kernel is the faster way to iterate an array: its time per step,
-// in us, against that of what would run otherwise.  Its own is the rounds of
-// workgroups times their plane steps, 0.35 us each and step (Wrap: 200^3 8.5,
-// 256^3 11.8, 384^3 30, 512^3 73.5 us; the edge cells of Remove and Reflect
-// make it 0.47 and 0.5, 2-byte storage 15% more).  zmarch2_kernel, from 2^21
-// cells, takes 1.06 us per 10^6 cells and 6 at least (f32 Wrap: 128^3 6.1, 200^3
-// 10.0, 256^3 17.5, 384^3 66, 512^3 162 us; 2-byte cells move half the bytes
-// and keep it); one launch per step below that 5 + 1.5 per 10^6 cells (32^3
-// 4.9, 100^3 7.9; here 3.9 and 4.5).
-inline bool zmarch_pays(int64_t n0, int64_t n1, int64_t n2, int bc, int es, const ZmGrid& grid, bool zmarch2) {
-  if (zmarch2 && es != 4) return false;
-  const double here = (bc == STH_WRAP ? 0.35 : (bc == STH_REMOVE ? 0.47 : 0.5)) * (es == 4 ? 1.0 : 1.15) *
-                      static_cast<double>(grid.time);
-  const double mcells = 1e-6 * static_cast<double>(n0) * static_cast<double>(n1) * static_cast<double>(n2);
-  const double other = zmarch2 ? (1.06 * mcells > 6.0 ? 1.06 * mcells : 6.0) : 5.0 + 1.5 * mcells;
-  return here < other;
-}
-
 template <typename S, int OPK, class Sh>
 void launch_zmarch(const MapParams& p, hipStream_t s) {
   const unsigned nb = static_cast<unsigned>(p.tiles_x) * p.tiles_y * p.tiles_z;

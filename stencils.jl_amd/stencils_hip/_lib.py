@@ -19,6 +19,7 @@ LIB_PATH = Path(os.environ.get("STENCILS_HIP_LIB", PKG_ROOT / "lib" / "libstenci
 EXPORTS = {
     "sth_version": (ctypes.c_int, []),
     "sth_last_error": (ctypes.c_char_p, []),
+    "sth_steps_kernel": (ctypes.c_char_p, []),
     "sth_ctx_create": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(ctypes.c_void_p)]),
     "sth_ctx_destroy": (ctypes.c_int, [ctypes.c_void_p]),
     "sth_alloc": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_size_t, ctypes.POINTER(ctypes.c_void_p)]),
@@ -136,6 +137,11 @@ def tuning_table(device: int = 0) -> dict:
 def set_variant(pattern: str = "", device: int = 0):
     """Force the first kernel variant whose name contains `pattern` ("" = tuner)."""
     check(lib().sth_set_variant(context(device), pattern.encode()))
+
+
+def steps_kernel() -> str:
+    """What this thread's last iteration ran its steps on ("single", "ymarch/8", ...)."""
+    return lib().sth_steps_kernel().decode()
 
 
 def context(device: int = 0):

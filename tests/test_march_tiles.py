@@ -42,7 +42,8 @@ def run(tmp_path_factory):
 
     def go(code):
         (d / "check.cpp").write_text(code)
-        subprocess.run(["g++", "-std=c++17", "-O1", f"-I{REPO / 'stencils.jl_amd' / 'csrc'}", str(d / "check.cpp"),
+        subprocess.run(["g++", "-std=c++17", "-O1", f"-I{REPO / 'stencils.jl_amd' / 'csrc'}",
+                        f"-I{REPO / 'include'}", str(d / "check.cpp"),
                         "-o", str(d / "check")], check=True)
         return subprocess.run([str(d / "check")], capture_output=True, text=True)
 
@@ -104,4 +105,63 @@ int main() {
 def test_plane_chunks_are_the_shortest(run):
     r = run(ZGRID)
     print(r.stdout)
+    assert r.returncode == 0, r.stdout
+
+
+COST = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "march_cost.hpp"
+
+using namespace sth;
+static int bad = 0;
+static void expect(bool ok, const char* what, long a = 0, long b = 0) {
+  if (!ok && ++bad <= 10) std::printf("%s (%ld, %ld)\n", what, a, b);
+}
+static MarchCall call(int64_t n0, int64_t n1, int dtype, int op, int L, int bc) {
+  return MarchCall{n0, n1, dtype, op, L, bc, true, true, false};
+}
+
+int main() {
+  // the launches of an iteration: all its steps, none longer than G, their number of the parity of their steps
+  for (int64_t G : {2, 4, 6, 8})
+    for (int64_t least : {1, 2})
+      for (int64_t n = 4; n <= 300; ++n) {
+        const StepLaunches l = march_cheapest(n, least, 5.0, StepKernel{G, 9.0, 0.5});
+        expect(l.singles >= least && l.singles < n, "single steps", G, n);
+        const int64_t gens = n - l.singles, f = march_launches(gens, G);
+        expect(f == l.multi && (f - gens) % 2 == 0, "launches", G, n);
+        int64_t left = gens;
+        for (int64_t i = 0; i < f; ++i) {
+          const int64_t g = march_share(i, f, left, G);
+          expect(g >= 1 && g <= G, "steps of a launch", G, n);
+          left -= g;
+        }
+        expect(left == 0, "steps left", G, n);
+      }
+  // as measured (us): see march_choose
+  expect(march_choose(call(262144, 16, STH_F64, STH_OP_MEAN, 9, STH_REFLECT), 6, 33, 1, 256).gens == 2, "few rows");
+  expect(march_choose(call(262144, 16, STH_F32, STH_OP_LAPLACIAN, 4, STH_REMOVE), 8, 7, 1, 256).gens != 8, "few rows, few steps");
+  expect(march_choose(call(1 << 21, 8, STH_F32, STH_OP_LAPLACIAN, 4, STH_WRAP), 8, 33, 1, 256).gens == 2, "8 rows");
+  expect(march_choose(call(16, 262144, STH_F32, STH_OP_MEAN, 9, STH_WRAP), 6, 33, 1, 256).gens == 0, "few columns");
+  const MarchChoice five = march_choose(call(300, 200, STH_F32, STH_OP_MEAN, 9, STH_WRAP), 6, 5, 1, 256);
+  expect(five.gens != 6 || five.singles == 2, "five steps: not in two long launches and a single step");
+  for (int64_t n : {512, 1024, 2048, 4096, 8192}) {
+    expect(march_choose(call(n, n, STH_F32, STH_OP_LAPLACIAN, 4, STH_WRAP), 8, 100, 1, 256).gens == 8, "f32 heat", n);
+    expect(march_choose(call(n, n, STH_F64, STH_OP_LAPLACIAN, 4, STH_WRAP), 8, 100, 1, 256).gens == 8, "f64 heat", n);
+    expect(march_choose(call(n, n, STH_F32, STH_OP_MEAN, 9, STH_REMOVE), 6, 100, 1, 256).gens == 6, "f32 mean", n);
+  }
+  // 3-D: three steps in one launch and three single ones, not three launches (64^3 f32, 6 steps: 60 us, 46 before)
+  for (int64_t n : {32, 64, 100})
+    expect(zmarch_singles(n, n, n, STH_WRAP, 4, zmarch_grid(n, n, n, 256), false, false, false, 6, 1) >= 3, "3-D, six steps", n);
+  for (int64_t n : {64, 100, 200, 256, 384})
+    expect(zmarch_singles(n, n, n, STH_WRAP, 4, zmarch_grid(n, n, n, 256), n >= 128, false, true, 100, 1) < 8, "3-D, 100 steps", n);
+  std::printf("%d bad\n", bad);
+  return bad != 0;
+}
+"""
+
+
+def test_launches_and_choices(run):
+    r = run(COST)
     assert r.returncode == 0, r.stdout
