@@ -165,3 +165,37 @@ int main() {
 def test_launches_and_choices(run):
     r = run(COST)
     assert r.returncode == 0, r.stdout
+
+
+LIFE = r"""
+#include <chrono>
+#include <cstdio>
+#include "lifep_shape.hpp"
+
+using namespace sth;
+
+int main() {
+  int bad = 0;
+  // more sizes than are remembered, each twice
+  for (int64_t i = 0; i < 3000; ++i) {
+    const int64_t n0 = 64 + 7 * i, n1 = 3 + (i * i) % 9000;
+    const LifepShape a = lifep_shape(n0, n1, i % 2 != 0, 256), b = lifep_shape(n0, n1, i % 2 != 0, 256),
+                     c = lifep_search(n0, n1, i % 2 != 0, 256);
+    const bool same = a.k == b.k && a.gens == b.gens && a.lpr_shift == b.lpr_shift && a.k == c.k && a.gens == c.gens &&
+                      a.lpr_shift == c.lpr_shift;
+    // a tile keeps at least one row, a rim word at least the bits it loses
+    if (!same || a.gens > kLifepMaxGens || (kLifepWaves << (6 - a.lpr_shift)) * a.k - 2 * a.gens < 1) ++bad;
+  }
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int i = 0; i < 1000; ++i) bad += lifep_shape(1501, 1333, true, 256).k < 1;
+  const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() / 1000;
+  std::printf("%d bad, %.2f us a call\n", bad, us);
+  return bad != 0 || us > 3.0;  // the search itself takes four times that
+}
+"""
+
+
+def test_life_shapes_are_remembered(run):
+    r = run(LIFE)
+    print(r.stdout)
+    assert r.returncode == 0, r.stdout
