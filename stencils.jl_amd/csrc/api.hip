@@ -2463,11 +2463,15 @@ int sth_jit_selftest(char* log, size_t cap) {
   };
   const int dts[] = {STH_BOOL, STH_U8, STH_I16, STH_I32, STH_I64, STH_F32, STH_F64, STH_BF16};
   for (int dt : dts) {
-    const std::string targs = std::string(jit_type_name(dt)) + ", " + std::to_string(STH_OP_MAX) +
-                              ", sth::jit::Shape, 4, 4";
-    one("#include \"stream_kernel.hpp\"\n" + jit_shape_source(6, &shape[0][0], 2, 2, 0) +
-            "namespace sth {\ntemplate __global__ void stream_kernel<" + targs + ">(MapParams);\n}\n",
-        "&sth::stream_kernel<" + targs + ">", "stream " + std::string(jit_type_name(dt)));
+    std::string src, expr;
+    jit_stream_source(dt, STH_OP_MAX, 6, &shape[0][0], 2, 2, 0, 4, 4, &src, &expr);
+    one(src, expr, "stream " + std::string(jit_type_name(dt)));
+  }
+  for (int ky : {4, 8}) {
+    std::string src, expr;
+    const int dt = ky == 4 ? STH_I8 : STH_U8;
+    jit_bytes_source(dt, ky == 4 ? STH_OP_MIN : STH_OP_MAX, 6, &shape[0][0], 2, 2, ky, &src, &expr);
+    one(src, expr, "bytes " + std::string(jit_type_name(dt)) + " " + std::to_string(ky));
   }
   struct M {
     int dt, op;
@@ -2505,13 +2509,19 @@ int sth_jit_selftest(char* log, size_t cap) {
       one(src, expr, std::string("fused multi ") + jit_type_name(m.dt) + " " + m.items);
     }
   }
-  const int fdt[][3] = {{STH_I32, STH_OP_MAX, 2}, {STH_I64, STH_OP_SUM, 2}, {STH_F32, STH_OP_SUM, 2},
-                        {STH_I16, STH_OP_MIN, 3}, {STH_I64, STH_OP_SUM, 3}, {STH_F64, STH_OP_MAX, 3}};
+  // multi-step kernels: type, fold, dimensions, boundary, steps per launch
+  const int fdt[][5] = {{STH_I32, STH_OP_MAX, 2, STH_WRAP, 8},    {STH_I32, STH_OP_MAX, 2, STH_REMOVE, 8},
+                        {STH_I32, STH_OP_MAX, 2, STH_REFLECT, 8}, {STH_I64, STH_OP_SUM, 2, STH_REMOVE, 8},
+                        {STH_I64, STH_OP_SUM, 2, STH_REFLECT, 2}, {STH_F32, STH_OP_SUM, 2, STH_WRAP, 2},
+                        {STH_I16, STH_OP_MIN, 2, STH_REFLECT, 4}, {STH_I16, STH_OP_MIN, 2, STH_REMOVE, 2},
+                        {STH_I16, STH_OP_MIN, 3, STH_WRAP, 2},    {STH_I64, STH_OP_SUM, 3, STH_REMOVE, 2},
+                        {STH_F64, STH_OP_MAX, 3, STH_REFLECT, 2}};
   for (const auto& c : fdt) {
     std::string src, expr;
     jit_fused_source(c[0], c[1], c[2] == 3 ? 6 : 4, c[2] == 3 ? &vn3[0][0] : &vn2[0][0], 1, 1, c[2] == 3 ? 1 : 0, c[2],
-                     STH_WRAP, 2, &src, &expr);
-    one(src, expr, std::string("two-step ") + std::to_string(c[2]) + "-D " + jit_type_name(c[0]));
+                     c[3], c[4], &src, &expr);
+    one(src, expr, std::to_string(c[4]) + "-step " + std::to_string(c[2]) + "-D " + jit_type_name(c[0]) +
+                       " boundary " + std::to_string(c[3]));
   }
   {
     // Moore(1) in a 66-wide box, residues in some order

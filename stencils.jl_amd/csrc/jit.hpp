@@ -340,43 +340,57 @@ inline const JitKernel* jit_remembered(const JitRequest& r, Build&& build) {
   return k;
 }
 
-// The streaming kernel specialised to one shape (L offsets, x fastest, as
-// int8 triples) for storage type `dtype`, fold `opk`, V cells per lane and
-// KY rows per lane, loaded on the current device.
+// The source of the streaming kernel specialised to one shape (L offsets, x
+// fastest, as int8 triples) for storage type `dtype`, fold `opk`, V cells per
+// lane and KY rows per lane (false: no type name).
+inline bool jit_stream_source(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz, int v, int ky,
+                              std::string* src_out, std::string* expr_out) {
+  const char* tn = jit_type_name(dtype);
+  if (!tn) return false;
+  const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " +
+                            std::to_string(v) + ", " + std::to_string(ky);
+  *src_out = "#include \"stream_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, rz) +
+             "namespace sth {\ntemplate __global__ void stream_kernel<" + targs + ">(MapParams);\n}  // namespace sth\n";
+  *expr_out = "&sth::stream_kernel<" + targs + ">";
+  return true;
+}
+
+// It, loaded on the current device.
 inline const JitKernel* jit_stream_kernel(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int rz,
                                           int v, int ky, std::string* why) {
   const JitRequest request = JitRequest('s').add(dtype).add(opk).add(rx).add(ry).add(rz).add(v).add(ky).add(offs3, 3 * static_cast<size_t>(L));
   return jit_remembered(request, [&]() -> const JitKernel* {
-    const char* tn = jit_type_name(dtype);
-    if (!tn) {
+    std::string src, expr;
+    if (!jit_stream_source(dtype, opk, L, offs3, rx, ry, rz, v, ky, &src, &expr)) {
       *why = "no type name";
       return nullptr;
     }
-    const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " +
-                              std::to_string(v) + ", " + std::to_string(ky);
-    const std::string src = "#include \"stream_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, rz) +
-                            "namespace sth {\ntemplate __global__ void stream_kernel<" + targs +
-                            ">(MapParams);\n}  // namespace sth\n";
-    return jit_load(src, "&sth::stream_kernel<" + targs + ">",
-                    "stream" + std::to_string(v) + "x" + std::to_string(ky), why);
+    return jit_load(src, expr, "stream" + std::to_string(v) + "x" + std::to_string(ky), why);
   });
 }
 
 // The one-byte extremes kernel (bytes_kernel) specialised to one shape.
+inline bool jit_bytes_source(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int ky,
+                             std::string* src_out, std::string* expr_out) {
+  const char* tn = jit_type_name(dtype);
+  if (!tn) return false;
+  const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " + std::to_string(ky);
+  *src_out = "#include \"bytes_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, 0) +
+             "namespace sth {\ntemplate __global__ void bytes_kernel<" + targs + ">(MapParams);\n}  // namespace sth\n";
+  *expr_out = "&sth::bytes_kernel<" + targs + ">";
+  return true;
+}
+
 inline const JitKernel* jit_bytes_kernel(int dtype, int opk, int L, const int8_t* offs3, int rx, int ry, int ky,
                                          std::string* why) {
   const JitRequest request = JitRequest('b').add(dtype).add(opk).add(rx).add(ry).add(ky).add(offs3, 3 * static_cast<size_t>(L));
   return jit_remembered(request, [&]() -> const JitKernel* {
-    const char* tn = jit_type_name(dtype);
-    if (!tn) {
+    std::string src, expr;
+    if (!jit_bytes_source(dtype, opk, L, offs3, rx, ry, ky, &src, &expr)) {
       *why = "no type name";
       return nullptr;
     }
-    const std::string targs = std::string(tn) + ", " + std::to_string(opk) + ", sth::jit::Shape, " + std::to_string(ky);
-    const std::string src = "#include \"bytes_kernel.hpp\"\n" + jit_shape_source(L, offs3, rx, ry, 0) +
-                            "namespace sth {\ntemplate __global__ void bytes_kernel<" + targs +
-                            ">(MapParams);\n}  // namespace sth\n";
-    return jit_load(src, "&sth::bytes_kernel<" + targs + ">", "bytes" + std::to_string(ky), why);
+    return jit_load(src, expr, "bytes" + std::to_string(ky), why);
   });
 }
 
