@@ -600,9 +600,16 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
                            reach[2] == 0 && n[0] >= kBytesMinN0 && n[0] <= (int64_t(1) << 30) && L > 0;
         if (bytes) {
           v = kBytesV;
-          // eight rows per lane re-read fewer, where four waves per SIMD are
-          // left and their registers suffice: the same call 58 us, 62 with four
-          ky = rmax <= 2 && cells >= (int64_t(1) << 25) ? 8 : 4;
+          // Eight rows per lane re-read fewer, which pays where rows are read
+          // for two rows on either side and the fold is most of the work, and
+          // four waves per SIMD are left (kernel times: 5 x 5 maximum of
+          // 8192^2 39.9 us, 42.7 with four; 5793^2 22.3, 24.2; 64 x 2^19 31.2,
+          // 36.9).  Else four: 3 x 3 maximum of 16384^2 104.7, 112.6 with
+          // eight; six offsets of reach 2 107.4, 115.0; and on few rows, 2^22
+          // x 16, 5 x 5 41.8, 50.1.  (STH_BYTES_KY, read per call: 4 or 8
+          // rows, to test and compare them)
+          ky = rmax <= 2 && reach[1] == 2 && L >= 16 && n[1] >= 32 && cells >= (int64_t(1) << 25) ? 8 : 4;
+          if (const char* e = std::getenv("STH_BYTES_KY")) ky = rmax <= 2 && std::atoi(e) == 8 ? 8 : 4;
         }
         std::vector<int8_t> o8(3 * L);
         for (int i = 0; i < 3 * L; ++i) o8[i] = static_cast<int8_t>(offs3[i]);
