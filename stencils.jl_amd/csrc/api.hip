@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdlib>
@@ -248,8 +249,19 @@ bool offsets_equal(const int8_t* tbl, int L, const std::vector<int>& offs3) {
   return true;
 }
 
-// Compute units of an MI355X: what the marching kernels' grids are cut for.
-constexpr int kCus = 256;
+// Compute units of the current device (a partition of an MI355X has fewer
+// than its 256): what the marching kernels' grids are cut for.
+int device_cus() {
+  static std::atomic<int> known[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = known[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    known[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
 
 // Bytes from an array descriptor's base to the end of its last cell.
 int64_t zm2_extent(const DevArr& a, int64_t esize) {
@@ -672,6 +684,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
                      (bc == STH_WRAP || bc == STH_REMOVE || bc == STH_REFLECT) &&
                      zm2_extent(pl.p.src, dtype_size(sdt)) < kZm2MaxBytes &&
                      zm2_extent(pl.p.dst, dtype_size(odt)) < kZm2MaxBytes;
+  const int cus = multi ? device_cus() : 0;
   const char* const wanted = multi ? std::getenv("STH_STEPS_KERNEL") : nullptr;
 
   // 3-D: up to four steps for star stencils of 4-byte values (zmarch_kernel),
@@ -690,7 +703,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       if (wanted && std::strcmp(wanted, e.name) != 0) continue;
       if (e.any) {
         if (n[0] < kZmMinCells || n[1] < kZmMinCells || n[2] < kZmMinCells) continue;
-        const ZmGrid grid = zmarch_grid(n[0], n[1], n[2], kCus);
+        const ZmGrid grid = zmarch_grid(n[0], n[1], n[2], cus);
         const int64_t singles =
             wanted ? least_singles
                    : zmarch_singles(n[0], n[1], n[2], bc, dtype_size(sdt), grid, big, least_singles > 1,
@@ -767,7 +780,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
       } else if (fuse2d_min < 0) {
         const MarchCall call{n[0], n[1], sdt, op->kind, L, bc,
                              rows_on(pl.p.src, es2, 16) && rows_on(pl.p.dst, es2, 16), built[0] != nullptr, least_singles > 1};
-        c = march_choose(call, most, steps, least_singles, kCus);
+        c = march_choose(call, most, steps, least_singles, cus);
       }
       if (c.gens && built[0]) {
         pl.fn_fused = built[c.gens == kYmShortGens]->fn;
@@ -785,7 +798,7 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
         pl.fused_any = 1;
         pl.fused_singles = c.singles;
         pl.fused_name = ymarch_name(c.gens);
-        const YmGrid grid = ymarch_grid(n[0], n[1], static_cast<int>(16 / es2), c.gens, kCus);
+        const YmGrid grid = ymarch_grid(n[0], n[1], static_cast<int>(16 / es2), c.gens, cus);
         pl.fused_tiles_x = static_cast<int32_t>(grid.tx);
         pl.fused_tiles_y = static_cast<int32_t>(grid.ty);
         pl.fused_tiles_z = static_cast<int32_t>(grid.rows);
