@@ -1146,10 +1146,14 @@ bool batch_merge_enabled() {
 // The 2-D groups of each element type that has several become one, which the
 // kernel of every 2-D variant runs, longest stencils first -- unless they are
 // large enough to fill the device one after another: a launch and its tail
-// cost about 6 us, the merged kernel about 0.6 ns per tile (9 variants of f32:
-// 1000 tiles each 95 us merged, 167 apart; 33000 each 2.96 ms merged, 2.78
-// apart).
-constexpr int64_t kMergeTiles = 8192;
+// cost about 6 us, while the merged kernel has the registers of its longest
+// variant and fewer waves, 8-byte types the fewest.  Tiles per variant up to
+// which it is the faster one, with 2, 4 and 9 variants (us merged / apart):
+// f32 4096 tiles 162 / 195, 319 / 361, 674 / 720, 16128 tiles 477 / 475, 925 /
+// 926, 1999 / 1877; f64 2048 tiles 92 / 120, 155 / 173, 358 / 351, 8192 tiles
+// 372 / 351, 633 / 603, 1358 / 1171; bf16 4096 tiles 290 / 322, 594 / 606,
+// 1268 / 1236, 8064 tiles 448 / 452, 894 / 844, 1885 / 1725.
+int64_t merge_tiles(int dtype) { return dtype_size(dtype) == 8 ? 3072 : dtype_size(dtype) == 2 ? 4096 : 8192; }
 void merge_groups(BatchGroups* groups, std::map<int64_t, double>* cost) {
   std::map<int64_t, std::vector<int64_t>> keys;  // element type -> its 2-D groups
   for (const auto& e : batch_kernels()) {
@@ -1162,7 +1166,7 @@ void merge_groups(BatchGroups* groups, std::map<int64_t, double>* cost) {
     int64_t tiles = 0;
     for (int64_t k : ks)
       for (const BatchJob& j : (*groups)[k]) tiles += static_cast<int64_t>(j.tiles_x) * j.tiles_y * j.tiles_z;
-    if (tiles > kMergeTiles * static_cast<int64_t>(ks.size())) continue;
+    if (tiles > merge_tiles(static_cast<int>(kv.first)) * static_cast<int64_t>(ks.size())) continue;
     auto per_cell = [&](int64_t k) {
       double cells = 0;
       for (const BatchJob& j : (*groups)[k]) cells += static_cast<double>(j.src.n0) * j.src.n1 * j.src.n2;
