@@ -479,9 +479,11 @@ int make_plan(const sth_array* src, const sth_array* dst, const sth_stencil* st,
     }
     group = std::string(conway ? "life_conway" : "life_table") + (sdt == STH_BOOL ? "_bool" : "_u8") + bucket;
     if (halo_pad && bc != STH_USE) {
-      // map boundaries in registers and refresh the source halo in the same launch
+      // map boundaries in registers and refresh the source halo, of one cell, in
+      // the same launch; a wider one (eight neighbours of a stencil that says
+      // it reaches further) has its own
       p.read_halo = 0;
-      p.fuse_halo = 1;
+      p.fuse_halo = src->halo == 1;
     }
     // Conway's rule under Wrap / Remove / Reflect on grids below 2 GiB:
     // several generations per launch with one bit per cell (lifeb_kernel)
