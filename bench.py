@@ -67,19 +67,18 @@ def kernel_launch_us(sh, torch, S, rule, launches: int = 200):
     return S, e0.elapsed_time(e1) / launches * 1e3
 
 
-# Generations one launch of the steady-state Life kernel advances (the
-# library's default; STH_LIFEB_G overrides it there and here).
-LIFE_GENS = int(os.environ.get("STH_LIFEB_G", "8"))
+# Generations whose time and traffic the headline's roofline gives, and the
+# generations of the launch that profiles/lifep_kernel_gol_8192.md measured.
+LIFE_GENS = 8
+LIFE_PROFILED_GENS = 32
 
 
 def fused_launch_us(sh, torch, S, rule, gens: int, m1: int = 1, m2: int = 5):
-    """Average duration of one launch of the multi-generation Life kernel
-    (`gens` generations per launch).  A call of 3 + 32 gens m generations
-    runs one eager step, m replays of the captured 16-unit graph (32 fused
-    launches each) and the same 2-step tail for every m, so the difference
-    of two such calls, timed between HIP events on the launch stream, is
-    (m2 - m1) x 32 launches of the kernel alone.  Both calls' graphs are
-    captured before timing."""
+    """Average duration of `gens` generations of the multi-generation Life
+    kernel, without the ends of a call: the difference of two calls of
+    3 + 32 gens m generations, timed between HIP events on the launch stream,
+    is (m2 - m1) x 32 times as many.  Both calls' graphs are captured before
+    timing."""
     stream = torch.cuda.current_stream()
     steps = lambda m: 3 + 32 * gens * m  # noqa: E731
     for m in (m1, m2, m1, m2):  # capture both keys at both buffer parities
@@ -619,8 +618,8 @@ def bench_served(sh, torch, n: int = 120, budget: int = 2 << 30):
 def bench_heat_iterate(sh, torch, n: int = 512, steps: int = 200):
     """3-D heat iteration (VonNeumann(1,3) Laplacian(0.15), Wrap, n^3) as
     `steps` hipGraph-replayed steps: several steps per launch (zmarch_kernel or zmarch2_kernel)
-    against one streaming step per launch (STH_NO_FUSE).  The two-step
-    kernel's roofline counts both steps' algorithmic bytes per launch."""
+    against one streaming step per launch (STH_NO_FUSE).  The achieved rates
+    count every step's algorithmic bytes."""
     f = sh.Laplacian(0.15)
     dev = torch.device("cuda", torch.cuda.current_device())
     stream = torch.cuda.current_stream()
@@ -630,7 +629,7 @@ def bench_heat_iterate(sh, torch, n: int = 512, steps: int = 200):
         A.copy_(torch.rand((n,) * 3, device=dev).to(tdt))
         S = sh.SwitchingStencilArray(A, sh.VonNeumann(1, 3), boundary=sh.Wrap())
         t = {}
-        for key, fl in (("two_step", 0), ("one_step", sh._abi.NO_FUSE)):
+        for key, fl in (("multi_step", 0), ("one_step", sh._abi.NO_FUSE)):
             S = sh.mapstencil_steps(f, S, 8, flags=sh._abi.ASYNC | fl)
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             torch.cuda.synchronize()
@@ -641,15 +640,15 @@ def bench_heat_iterate(sh, torch, n: int = 512, steps: int = 200):
             t[key] = e0.elapsed_time(e1) / steps * 1e3  # us per step
         es = A.element_size()
         cells = n ** 3
-        launch_us = 2 * t["two_step"]
-        res[name] = {"two_step_us_per_step": t["two_step"], "one_step_us_per_step": t["one_step"],
-                     "speedup": t["one_step"] / t["two_step"],
-                     "cell_steps_per_s": cells / (t["two_step"] * 1e-6),
-                     "two_step_roofline": {"bytes_per_launch": 2 * 2 * es * cells, "avg_launch_us": launch_us,
-                                           "achieved_gbs": 2 * 2 * es * cells / (launch_us * 1e-6) / 1e9},
+        res[name] = {"multi_step_us_per_step": t["multi_step"], "one_step_us_per_step": t["one_step"],
+                     "speedup": t["one_step"] / t["multi_step"],
+                     "cell_steps_per_s": cells / (t["multi_step"] * 1e-6),
+                     "multi_step_achieved_gbs": 2 * es * cells / (t["multi_step"] * 1e-6) / 1e9,
                      "one_step_achieved_gbs": 2 * es * cells / (t["one_step"] * 1e-6) / 1e9}
         if name == "f32" and n == 512:
-            res[name]["two_step_roofline"]["traffic"] = profiled_traffic("zmarch2_kernel_heat_512.md")
+            # (the profile is of a launch of four steps)
+            traffic = profiled_traffic("zmarch_kernel_heat_512.md")
+            res[name]["multi_step_traffic_per_step"] = traffic and traffic // 4
             res[name]["one_step_traffic"] = profiled_traffic("zmarch1_kernel_heat_512.md")
         del A, S
         torch.cuda.empty_cache()
@@ -708,7 +707,7 @@ def bench_heat_iterate_2d(sh, torch, steps: int = 100):
     """2-D heat iteration (VonNeumann(1) Laplacian(0.2), Wrap) as `steps`
     hipGraph-replayed steps: several steps per launch (ymarch_kernel) against one
     streaming step per launch (STH_NO_FUSE); f32 and bf16 on 16384^2, f64 on
-    8192^2 (a 16384^2 f64 grid is past the two-step kernel's 2 GiB offsets)."""
+    8192^2 (a 16384^2 f64 grid is past the multi-step kernel's 2 GiB offsets)."""
     f = sh.Laplacian(0.2)
     dev = torch.device("cuda", torch.cuda.current_device())
     stream = torch.cuda.current_stream()
@@ -719,7 +718,7 @@ def bench_heat_iterate_2d(sh, torch, steps: int = 100):
         A.copy_(torch.rand((n, n), device=dev).to(tdt))
         S = sh.SwitchingStencilArray(A, sh.VonNeumann(1), boundary=sh.Wrap())
         t = {}
-        for key, fl in (("two_step", 0), ("one_step", sh._abi.NO_FUSE)):
+        for key, fl in (("multi_step", 0), ("one_step", sh._abi.NO_FUSE)):
             S = sh.mapstencil_steps(f, S, 8, flags=sh._abi.ASYNC | fl)
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             torch.cuda.synchronize()
@@ -729,15 +728,39 @@ def bench_heat_iterate_2d(sh, torch, steps: int = 100):
             torch.cuda.synchronize()
             t[key] = e0.elapsed_time(e1) / steps * 1e3
         es = A.element_size()
-        res[name] = {"n": n, "two_step_us_per_step": t["two_step"], "one_step_us_per_step": t["one_step"],
-                     "speedup": t["one_step"] / t["two_step"],
-                     "two_step_achieved_gbs": 2 * 2 * es * n * n / (2 * t["two_step"] * 1e-6) / 1e9,
+        res[name] = {"n": n, "multi_step_us_per_step": t["multi_step"], "one_step_us_per_step": t["one_step"],
+                     "speedup": t["one_step"] / t["multi_step"],
+                     "multi_step_achieved_gbs": 2 * es * n * n / (t["multi_step"] * 1e-6) / 1e9,
                      "one_step_achieved_gbs": 2 * es * n * n / (t["one_step"] * 1e-6) / 1e9}
         if name == "f32":
-            res[name]["two_step_traffic"] = None
+            # (the profile is of a launch of eight steps)
+            traffic = profiled_traffic("ymarch_kernel_heat2d_16384.md")
+            res[name]["multi_step_traffic_per_step"] = traffic and traffic // 8
         del A, S
         torch.cuda.empty_cache()
     return res
+
+
+def result_line(out: dict) -> dict:
+    """The headline with its roofline, the plain paths beside it, and the
+    batched and served workloads' figures."""
+    line = {k: v for k, v in out.items() if k not in ("cpu_baseline", "configs", "single_generation_kernel")}
+    line["config"] = {"workload": "game-of-life 8192x8192 UInt8, Moore(1), Wrap, Halo, B3/S23, all steps in one "
+                                  "sth_iterate call", "cells": out["config"]["cells"], "step": "one generation"}
+    line["roofline"] = {k: out["roofline"][k] for k in ("bound", "achieved", "peak", "unit", "frac", "traffic",
+                                                        "bytes_per_launch", "avg_launch_us", "stream_copy_gbs")}
+    line["roofline"]["note"] = "algorithmic bytes; several generations per launch, so frac may exceed 1"
+    line["plain_per_step"] = {"value": out["plain_per_step"]["value"], "unit": "cells/s"}
+    if "cpu_baseline" in out:
+        line["cpu_baseline"] = {k: v for k, v in out["cpu_baseline"].items() if isinstance(v, (int, float))}
+    if "configs" in out:
+        b, v = out["configs"]["batched_uneven"], out["configs"]["served_heat_3d"]
+        line["batched"] = {"cells_per_s": b["batched"]["cells_per_s"], "vs_c_loop": b["speedup_vs_c_loop"],
+                           "vs_blocking_calls": b["speedup_vs_blocking_calls"]}
+        line["served"] = {"cell_steps_per_s": v["f32"]["cell_steps_per_s"], "p50_ms": v["f32"]["p50_s"] * 1e3,
+                          "p99_ms": v["f32"]["p99_s"] * 1e3,
+                          "vs_plain": {k: v["served_vs_serial"][k] for k in ("throughput", "p99_latency")}}
+    return line
 
 
 def main():
@@ -799,6 +822,7 @@ def main():
     # roofline is that of LIFE_GENS generations, timed on their own.
     S, launch_us = fused_launch_us(sh, torch, S, rule, LIFE_GENS)
     bytes_per_launch = LIFE_GENS * bytes_per_step
+    life_traffic = profiled_traffic("lifep_kernel_gol_8192.md")
     achieved = bytes_per_launch / (launch_us * 1e-6) / 1e9
     S, plain_launch_us = kernel_launch_us(sh, torch, S, rule)
     # measured stream-copy bandwidth on the same bytes (one read + one write)
@@ -838,13 +862,14 @@ def main():
                                "launched directly below)", "cells": cells, "step": "one generation"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": None,
+                     "traffic": life_traffic and life_traffic * LIFE_GENS // LIFE_PROFILED_GENS,
                      "kernel": f"lifep_kernel: {LIFE_GENS} generations of it (a launch runs up to 32), one bit "
                                "per cell",
                      "bytes_per_launch": bytes_per_launch, "avg_launch_us": launch_us,
                      "per_generation_us": gen_us,
                      "note": "algorithmic bytes count 2 B per cell and generation (temporal-blocking "
-                             "savings excluded), so frac may exceed 1",
+                             "savings excluded), so frac may exceed 1; traffic is the HBM bytes they move "
+                             "(rocprofv3 FETCH_SIZE x2 + WRITE_SIZE, a quarter of a 32-generation launch)",
                      "stream_copy_gbs": copy_gbs},
         "single_generation_kernel": {
             "kernel": "life_kernel<KY tuned, B3/S23>: one generation per launch (graph steps without temporal blocking)",
@@ -868,7 +893,10 @@ def main():
                           "scatter_downhill": bench_scatter(sh, torch),
                           "runtime_offsets": bench_runtime(sh, torch),
                           "iterate_batch_uneven": bench_iterate_batch(sh, torch)}
-    print(json.dumps(out), flush=True)
+    # the measured workloads in full go to stderr; the result line stays short
+    # enough to be read back from the end of a log
+    print(json.dumps(out), file=sys.stderr, flush=True)
+    print(json.dumps(result_line(out)), flush=True)
 
 
 if __name__ == "__main__":
