@@ -22,8 +22,9 @@ __device__ __forceinline__ float bf16_to_float(uint16_t b) {
 }
 // Round-to-nearest-even f32 -> bf16; NaN stays NaN (quiet bit forced): one
 // v_cvt_pk_bf16_f32, whose result equals the integer formulation
-// (x + 0x7fff + lsb) >> 16 for every one of the 2^32 inputs.  Six VALU
-// operations less per cell: bf16 Gaussian 7 x 7, 16384^2, 556 -> 517 us.
+// (x + 0x7fff + lsb) >> 16 (compared for all 2^32 inputs on a gfx950, NaN
+// patterns included; the tests cover sums of 4 x 65536).  bf16 Gaussian
+// 7 x 7, 16384^2: 72.2 -> 66.0 vector operations per cell, 556 -> 517 us.
 __device__ __forceinline__ uint16_t float_to_bf16(float f) {
   return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
