@@ -1,5 +1,7 @@
-"""The tiles of the marching kernels (csrc/march_tiles.hpp), compiled for the
-host: every cell belongs to one at least."""
+"""The host side of the multi-step kernels, compiled for the CPU: the tiles of
+the marching kernels (csrc/march_tiles.hpp: every cell belongs to one at least),
+the launches of an iteration and their choice (csrc/march_cost.hpp), and the
+tile shapes of the packed Life kernel (csrc/lifep_shape.hpp)."""
 import subprocess
 
 import pytest
